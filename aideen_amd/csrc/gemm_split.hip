@@ -368,7 +368,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN >= 8) ? 1 : 2) void k_ge
     }
 }
 
-// Skinny GEMM (at most 32 rows: one position of every sequence, a decode step).  There the
+// Skinny GEMM (the LM head at most 32 rows, the other products at most ATTN_FUSE_ROWS, which may
+// carry a fused stage: a decode step).  There the
 // ring kernel's serial k loop (one barrier per 16-K slice) is the whole cost, so here a
 // workgroup of KW waves owns a 32 x (32 WTN) output block and wave w multiplies its own K range
 // [w K/KW, (w+1) K/KW) straight from global memory into registers, 64 K values per step:
@@ -655,6 +656,163 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_skinny(GemmParams p) {
     epilogue_t<ROLE, 1, WTN, 1, 1>(p, acc, M, s, 0, n0, osc, am_v, am_i);
 }
 
+// K-sliced GEMM for grids that leave most of the chip idle (a few hundred rows or fewer, see
+// pick_tiles).  There the ring kernel is bound by the chain of its k loop, about 0.25 us per 16-K
+// slice however small the tile and however deep the ring (barrier, LDS reads, split, MFMAs: 10-18
+// us for K = 512 at 0.7 us of matrix work).  Here nothing is shared in the k loop, so it has no
+// barrier: a workgroup of KW waves owns a 32 WTM x 32 WTN output block, wave w multiplies the w-th
+// share of the 16-K steps straight from global memory, with U steps' loads in flight, and the KW
+// partial blocks are exchanged through LDS once, each wave then summing (in wave order) and storing
+// 1/KW of the block.  Lane (q = lane & 31, g = lane >> 5) loads K values [8g, 8g + 8) of a step of
+// A row q and B row q: one contiguous kilobyte of B per load, half lines of A.
+// Measured in back-to-back launches, K = 512, 8 slots, against the tiles used before: W_o at 64 rows 17.5 -> 5.3 us, at 256 rows 17.8 -> 10.2; Q|K|V at 64 rows 18.8 -> 9.6;
+// at 24 rows W_o 5.2 -> 4.9 and Q|K|V 6.7 -> 6.0 (the few-row kernel above).
+template <typename T, int TERMS, int KW, int WTM, int WTN>
+__global__ __launch_bounds__(64 * KW, KW == 8 ? 4 : (WTM == 2 ? 2 : 4)) void k_gemm_ks(GemmParams p) {
+    typedef typename Vec8<T>::type V8;
+    constexpr int U = 2;
+    constexpr int NE = WTM * WTN * 16;  // accumulators per lane
+    static_assert(NE % KW == 0, "the block's rows split evenly over the waves");
+    constexpr int BMt = 32 * WTM, BNt = 32 * WTN;
+    __shared__ float red[KW][NE][64];
+    const int nM = (p.M + BMt - 1) / BMt, nN = (p.N + BNt - 1) / BNt;
+    const int M = p.m_count ? min(*p.m_count, p.M) : p.M;
+    int s, mt, nt;
+    map_block(blockIdx.x, nM * nN * p.S, nM, nN, s, mt, nt);
+    const int m0 = mt * BMt, n0 = nt * BNt;
+    if (m0 >= M) return;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int q = lane & 31, g = lane >> 5;
+    const int steps = p.K / BK;
+    const int sb = wave * steps / KW, se = (wave + 1) * steps / KW;  // this wave's steps
+    // rows past M read row 0, column groups past N group 0 (their outputs are not stored)
+    const float *ap[WTM];
+#pragma unroll
+    for (int i = 0; i < WTM; ++i) {
+        const int m = m0 + 32 * i + q;
+        long ar = 0;
+        if (m < M) {
+            ar = p.a_idx ? (long)p.a_idx[m] : (long)m;
+            if (p.a_idx && (ar < 0 || ar >= p.a_idx_max)) {
+                if (p.err) atomicOr(p.err, ADN_DEVERR_TOKEN);
+                ar = 0;
+            }
+        }
+        ap[i] = p.A + ar * p.a_sm + (long)s * p.a_ss + 8 * g;
+    }
+    const T *bhp[WTN], *blp[WTN];
+#pragma unroll
+    for (int j = 0; j < WTN; ++j) {
+        const long grp = (n0 >> 5) + j;
+        const long off = (long)s * split_slot_stride(p) + (grp * 32 < p.N ? grp : 0) * (long)steps * 512 + q * 16 + 8 * g;
+        bhp[j] = reinterpret_cast<const T *>(p.Bhi) + off;
+        blp[j] = reinterpret_cast<const T *>(TERMS == 3 ? p.Blo : p.Bhi) + off;
+    }
+    float asc = p.a_scale, osc = p.out_scale;
+    if (p.a_absmax) {  // data-dependent A scale (power of two, never above the static one)
+        const float mx = __uint_as_float(*p.a_absmax);
+        if (mx > 0.0f) {
+            const float dyn = exp2f(floorf(log2f(p.a_headroom / mx)));
+            if (dyn < asc) {
+                osc *= asc / dyn;
+                asc = dyn;
+            }
+        }
+    }
+    floatx16 acc[WTM][WTN];
+#pragma unroll
+    for (int i = 0; i < WTM; ++i)
+#pragma unroll
+        for (int j = 0; j < WTN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    floatx4 a[U][WTM][2];
+    V8 bh[U][WTN], bl[U][WTN];
+    auto load = [&](int u, int st) {
+        const long sc = min(st, steps - 1);  // past the wave's share: a step that is not multiplied
+#pragma unroll
+        for (int i = 0; i < WTM; ++i) {
+            a[u][i][0] = *reinterpret_cast<const floatx4 *>(ap[i] + sc * BK);
+            a[u][i][1] = *reinterpret_cast<const floatx4 *>(ap[i] + sc * BK + 4);
+        }
+#pragma unroll
+        for (int j = 0; j < WTN; ++j) {
+            bh[u][j] = *reinterpret_cast<const V8 *>(bhp[j] + sc * 512);
+            if constexpr (TERMS == 3) bl[u][j] = *reinterpret_cast<const V8 *>(blp[j] + sc * 512);
+        }
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+        for (int i = 0; i < WTM; ++i) {
+            V8 ah, al;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float x = a[u][i][e >> 2][e & 3] * asc;
+                const T hv = (T)x;
+                ah[e] = hv;
+                if constexpr (TERMS == 3) al[e] = (T)(x - (float)hv);
+            }
+#pragma unroll
+            for (int j = 0; j < WTN; ++j) {
+                if constexpr (TERMS == 3) {
+                    acc[i][j] = mfma16(al, bh[u][j], acc[i][j]);
+                    acc[i][j] = mfma16(ah, bl[u][j], acc[i][j]);
+                }
+                acc[i][j] = mfma16(ah, bh[u][j], acc[i][j]);
+            }
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(u, sb + u);
+    int st = sb;
+    for (; st + U <= se; st += U) {
+        const bool more = st + U < se;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            multiply(u);
+            if (more) load(u, st + U + u);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (st + u < se) multiply(u);
+#pragma unroll
+    for (int i = 0; i < WTM; ++i)
+#pragma unroll
+        for (int j = 0; j < WTN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) red[wave][(i * WTN + j) * 16 + e][lane] = acc[i][j][e];
+    __syncthreads();
+    // accumulator el of the block: tile (i, j) = el / 16, and within it column q of row
+    // 8 (e / 4) + 4 g + e % 4, e = el % 16 (the MFMA's output layout)
+    constexpr int PE = NE / KW;
+    float v[PE], av[PE];
+    bool ok[PE];
+    long off[PE];
+#pragma unroll
+    for (int x = 0; x < PE; ++x) {
+        const int el = wave * PE + x, e = el & 15, i = (el >> 4) / WTN, j = (el >> 4) % WTN;
+        const int m = m0 + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3), n = n0 + 32 * j + q;
+        ok[x] = m < M && n < p.N;
+        off[x] = (long)m * p.c_sm + (long)s * p.c_ss + n;
+        av[x] = 0.0f;
+        if (p.epi == EPI_BIAS && ok[x] && n < p.bias_n) av[x] = p.bias[(long)s * p.bias_ss + n];
+        if (p.epi == EPI_ADD_A && ok[x]) av[x] = p.A[(long)m * p.a_sm + (long)s * p.a_ss + n];
+    }
+#pragma unroll
+    for (int x = 0; x < PE; ++x) {
+        const int el = wave * PE + x;
+        v[x] = red[0][el][lane];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) v[x] += red[w][el][lane];
+        v[x] = v[x] * osc + av[x];
+    }
+#pragma unroll
+    for (int x = 0; x < PE; ++x)
+        if (ok[x]) p.C[off[x]] = v[x];
+}
+
 // Weight split at upload: hi = T(w * scale), lo = T(w * scale - hi), from [S][N][K] fp32 into
 // the blocked layout: per slot, rows in groups of 32 (N padded to a multiple of 32 with zeros),
 // each group's K in blocks of 16, a block (32 rows x 16 halves, 1 KB) contiguous and row-major:
@@ -700,71 +858,96 @@ void launch_skinny(const GemmParams &p, int kw, hipStream_t st) {
     }
 }
 
+// Tiles of a GEMM below the 256x256 range: the configuration with the least a + b * (its blocks),
+// in us for K = 512, a fit to measured back-to-back launches of 8-slot products at 5 to 1000 rows
+// and N = 64 to 1536 (other K scale all of them alike).  a is the latency of one block's chain,
+// b the chip's time per block once the blocks outnumber the CUs:
+//   32x32   K-sliced over 8 waves   256 blocks  5.2 us,  768 blocks 10.0
+//   32x64   K-sliced over 4 waves   256 blocks  7.0 us,  768 blocks 14.1
+//   64x64   K-sliced over 4 waves   256 blocks 10.4 us,  768 blocks 23.6
+//   64x128  ring, waves of 32x64    256 blocks 14.1 us,  864 blocks 34.2
+//   128x128 ring, waves of 32x128   256 blocks 19.8 us,  768 blocks 44.2
+enum TilePick { TP_KS32, TP_KS32X64, TP_KS64, TP_R64X128, TP_R128 };
+TilePick pick_tiles(int M, int N, int S) {
+    static const struct {
+        int bm, bn;
+        float a, b;
+    } cf[] = {{32, 32, 3.0f, 0.0101f}, {32, 64, 4.0f, 0.0135f}, {64, 64, 5.0f, 0.0255f}, {64, 128, 10.0f, 0.0285f},
+              {128, 128, 13.0f, 0.041f}};
+    int best = 0;
+    float least = INFINITY;
+    for (int i = 0; i < 5; ++i) {
+        const float n = (float)((M + cf[i].bm - 1) / cf[i].bm) * (float)((N + cf[i].bn - 1) / cf[i].bn) * (float)S;
+        const float t = cf[i].a + cf[i].b * n;
+        if (t < least) {
+            least = t;
+            best = i;
+        }
+    }
+    return (TilePick)best;
+}
+
+int tiles(const GemmParams &p, int bm, int bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.S; }
+
+// The LM head below the 256x256 range, its blocks holding whole arg-max partials (128 columns):
+// 64x256 blocks of 32x128 waves, each A fragment split once per four column tiles (V = 50257,
+// K = 512: 64 rows 38.5 -> 23 us, 128 rows 38 -> 33, 531 rows 168 -> 138, 900 rows 263 -> 231
+// against the 128x128 blocks of 64x64 waves used before); a head too narrow to fill the chip takes
+// 64x128 blocks of 32x64 waves (V = 65, K = 192: 15.8 -> 9.8 us).
+template <typename T, int TERMS>
+void launch_lm_mid(const GemmParams &p, hipStream_t st) {
+    const int wide = tiles(p, 64, 256);
+    if (wide >= 64)
+        hipLaunchKernelGGL((k_gemm_split<ROLE_LMHEAD, T, TERMS, 1, 4, 2, 2, 4>), dim3(wide), dim3(256), 0, st, p);
+    else
+        hipLaunchKernelGGL((k_gemm_split<ROLE_LMHEAD, T, TERMS, 1, 2, 2, 2, 4>), dim3(tiles(p, 64, 128)), dim3(256), 0,
+                           st, p);
+}
+
 // Tile configurations (WTM, WTN, WGM, WGN, STAGES): GEMMs with M >= 1024 and N >= 512 use
-// 256x256 blocks of 8 waves (one workgroup per CU, 128 KB of LDS ring); the rest 128x128 blocks
-// of 4 waves (two workgroups per CU) so that their grids still cover the chip.  The 256x256
-// configuration runs persistent (one resident workgroup per CU walking its share of tiles, the
-// next tile's first slices loaded during the epilogue); the smaller ones launch a workgroup per
-// tile, whose short k loops would otherwise wait on the previous tile's stores.
+// 256x256 blocks of 8 waves (one workgroup per CU, 128 KB of LDS ring), persistent (one resident
+// workgroup per CU walking its share of tiles, the next tile's first slices loaded during the
+// epilogue); the rest take what pick_tiles says, a workgroup per tile.
 template <int ROLE, typename T, int TERMS>
 void launch_cfg(const GemmParams &p, hipStream_t st) {
+    if (p.M <= 0 || p.N <= 0 || p.S <= 0) return;
+    // K split over the waves of the few-row kernel, about two 64-K steps per wave (every K is a
+    // multiple of 64), each wave's K range whole 64-K steps
+    const int steps = p.K / 64;
+    int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
+    while (steps % kw) kw >>= 1;
     if constexpr (ROLE == ROLE_LMHEAD) {
-        if (p.M <= 32 && p.K % 64 == 0) {
+        if (p.M <= 32) {
             // skinny LM head (a decode step): 128-column blocks, the arg-max partials' width; at
             // a few rows 64-column blocks with partials per 64 columns (twice the workgroups on
-            // the weight stream, as for the other products); K split as below
-            const int steps = p.K / 64;
-            int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
-            while (steps % kw) kw >>= 1;
+            // the weight stream)
             if (gemm_lm_partial_cols(p.prec, p.M, p.K) == 64)
                 launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
             else
                 launch_skinny<ROLE, T, TERMS, 4>(p, kw, st);
             return;
         }
-    } else {
-        if (p.M <= 32 && p.K % 64 == 0) {
-            // skinny: K split over the waves of a workgroup, about two 64-K steps per wave;
-            // wide outputs take two column tiles per wave (each A fragment feeds both) except at
-            // a few rows, where twice the workgroups stream the weights sooner (decode Q|K|V at
-            // one row: 248 -> 238 us per token; at 32 rows the two-tile waves are 7% faster)
-            const int steps = p.K / 64;
-            int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
-            while (steps % kw) kw >>= 1;  // each wave's K range is whole 64-K steps
-            if constexpr (ROLE == ROLE_WO) {
-                if (p.attn_qkv) {  // the attention formed in the kernel (a few rows)
-                    launch_skinny<ROLE, T, TERMS, 1, true>(p, kw, st);
-                    return;
-                }
+    } else if (p.M <= ATTN_FUSE_ROWS) {
+        // a few rows: one 32-column tile per wave (decode Q|K|V at one row against two tiles:
+        // 248 -> 238 us per token).  The forms with a fused stage and the plain one are the same
+        // product bit for bit.
+        if constexpr (ROLE == ROLE_WO) {
+            if (p.attn_qkv) {  // the attention formed in the kernel
+                launch_skinny<ROLE, T, TERMS, 1, true>(p, kw, st);
+                return;
             }
-            if constexpr (ROLE == ROLE_QKV) {
-                if (p.upd_o) {  // the previous iteration's update formed in the kernel (a few rows)
-                    launch_skinny<ROLE, T, TERMS, 1, false, true>(p, kw, st);
-                    return;
-                }
+        }
+        if constexpr (ROLE == ROLE_QKV) {
+            if (p.upd_o) {  // the previous iteration's update formed in the kernel
+                launch_skinny<ROLE, T, TERMS, 1, false, true>(p, kw, st);
+                return;
             }
-            if (p.N >= 1024 && p.M > ATTN_FUSE_ROWS)
-                launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
-            else
-                launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
-            return;
         }
-        if (p.M <= 32) {
-            // skinny (at most 32 rows, e.g. one position of every sequence): 32x32 blocks of one
-            // wave, an 8-deep ring, so that the weight stream is spread over as many CUs as
-            // possible (an LM head with K not a multiple of 64 keeps the 128x128 tiles below: its
-            // arg-max partials are per 128 columns)
-            const int total = ((p.N + 31) / 32) * p.S;
-            if (total > 0)
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 1, 1, 1, 8>), dim3(total), dim3(64), 0, st, p);
-            return;
-        }
+        launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
+        return;
     }
-    const bool big = p.N >= 512 && p.M >= 1024;  // the configuration gemm_presplit_ok names
-    const int bm = big ? 256 : 128, bn = big ? 256 : 128;
-    const int total = ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.S;
-    if (total <= 0) return;
-    if (big) {
+    if (p.N >= 512 && p.M >= 1024) {  // the configuration gemm_presplit_ok names
+        const int total = tiles(p, 256, 256);
         // the roles whose A a producer writes pre-split (the slot mix, the LM head's normalised row)
         if constexpr (std::is_same<T, _Float16>::value && TERMS == 3 && (ROLE == ROLE_WO || ROLE == ROLE_LMHEAD)) {
             if (p.a_pre) {
@@ -773,22 +956,35 @@ void launch_cfg(const GemmParams &p, hipStream_t st) {
                 return;
             }
         }
-        if constexpr (ROLE == ROLE_QKV) {
+        if constexpr (ROLE == ROLE_QKV)
             // waves of 32 x 256 (8 down the block): each A row block is split by one wave only
             hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 8, 8, 1, 4>), dim3(ring_grid(total, 1)), dim3(512), 0, st,
                                p);
+        else
+            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4>), dim3(ring_grid(total, 1)), dim3(512), 0, st,
+                               p);
+        return;
+    }
+    if constexpr (ROLE == ROLE_LMHEAD) {
+        launch_lm_mid<T, TERMS>(p, st);
+    } else {
+        if (p.N <= 64 && p.M >= 1024) {
+            // narrow outputs (the carrier's projections, r + 2N = 64 columns): 128 x 64 blocks of two
+            // 64 x 64 waves, no zero-padded half tile
+            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 1, 4>), dim3(tiles(p, 128, 64)), dim3(128), 0, st, p);
             return;
         }
-        hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4>), dim3(ring_grid(total, 1)), dim3(512), 0, st,
-                           p);
+        switch (pick_tiles(p.M, p.N, p.S)) {
+            case TP_KS32: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 8, 1, 1>), dim3(tiles(p, 32, 32)), dim3(512), 0, st, p); break;
+            case TP_KS32X64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 1, 2>), dim3(tiles(p, 32, 64)), dim3(256), 0, st, p); break;
+            case TP_KS64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 2, 2>), dim3(tiles(p, 64, 64)), dim3(256), 0, st, p); break;
+            case TP_R64X128:
+                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 2, 2, 2, 4>), dim3(tiles(p, 64, 128)), dim3(256), 0, st, p);
+                break;
+            default:
+                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
+        }
     }
-    else if (p.N <= 64 && p.M >= 1024) {
-        // narrow outputs (the carrier's projections, r + 2N = 64 columns): 128 x 64 blocks of two
-        // 64 x 64 waves, no zero-padded half tile
-        const int t64 = ((p.M + 127) / 128) * ((p.N + 63) / 64) * p.S;
-        hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 1, 4>), dim3(t64), dim3(128), 0, st, p);
-    } else
-        hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 2, 4>), dim3(total), dim3(256), 0, st, p);
 }
 
 template <typename T, int TERMS>

@@ -1,0 +1,46 @@
+"""GEMM tile choices below 1024 rows (needs an MI355X): row and column counts on both sides of every
+block edge (32, 64, 128, 256) and slot counts that move the choice between the K-sliced and the ring
+kernels, every output against the oracle."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from aideen_amd import synth
+from aideen_amd.backend import GpuDeqBackend
+from test_gpu_parity import ATOL, RTOL
+
+pytestmark = pytest.mark.gpu
+
+# (d, H, V, B, T): the Q|K|V, W_o, signal, readout and LM-head products of B * T rows
+SHAPES = [
+    (64, 1, 65, 1, 5),      # fewer steps of K than waves
+    (64, 4, 31, 1, 31),     # one partial row block, one partial column block
+    (64, 16, 129, 1, 33),   # one row past a 32-row block
+    (192, 8, 65, 1, 128),   # whole blocks, narrow head
+    (128, 2, 257, 1, 129),  # one row and one column past a block
+    (320, 3, 300, 1, 65),   # K not a power of two, H not a power of two
+    (256, 8, 16500, 1, 97),  # a head wide enough for the 256-column blocks, its last partly filled
+    (192, 16, 513, 3, 171),  # 128-row ring blocks
+    (512, 8, 130, 1, 250),  # 64x64 K-sliced W_o, ring Q|K|V
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("flags", [0, synth.F_GEMM_BF16X3], ids=["f16x3", "bf16x3"])
+def test_tiles_match_oracle(shape, flags):
+    from oracle import pyoracle
+    d, H, V, B, T = shape
+    mc = synth.ModelConfig(d=d, H=H, V=V, N=4, max_iters=3, eps=0.0, qk_bias=True, flags=synth.F_SCAN_SELECTIVE | flags)
+    w = synth.make_token_sensitive_weights(mc)
+    toks = synth.make_tokens("uniform", B, T, V, seed=1)
+    be = GpuDeqBackend(mc, B, T)
+    be.upload_weights(w)
+    got = be.forward(toks)
+    be.close()
+    ref = pyoracle.Oracle(dataclasses.replace(mc, flags=synth.F_SCAN_SELECTIVE), w).forward(toks, nthreads=8)
+    for k in ("h_star", "pooled", "logits", "scan_y", "scan_state"):
+        np.testing.assert_allclose(got[k], ref[k], rtol=RTOL, atol=ATOL, err_msg=k)
+    # the fused arg-max is the last-max of the stored logits
+    lg = got["logits"].reshape(-1, V)
+    assert np.array_equal(got["argmax"].ravel(), V - 1 - np.argmax(lg[:, ::-1], axis=1))
