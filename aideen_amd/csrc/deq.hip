@@ -146,10 +146,16 @@ __device__ __forceinline__ void store_presplit_pair(float *row, int e0, const fl
     *reinterpret_cast<uint4 *>(reinterpret_cast<_Float16 *>(row) + (e0 >> 3) * 16 + (odd ? 8 : 0)) = out;
 }
 
-template <int H, int QA, int VEC>
+// H is the slot count, or (PAD) the power of two above it: the slots past D.H then read slot
+// D.H - 1 again, take no part in the softmax and store nothing.  The padded form replaced a kernel
+// that walked the slots at run time, one wave per query slot with a branch around each load: 6
+// slots of 320 at 4000 tokens 106 -> 40 us, 12 slots of 512 at 900 tokens 66 -> 54.
+template <int H, int QA, int VEC, bool PAD>
 __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, int k) {
     static_assert(QA * H <= 64, "the score butterfly leaves one score per lane: at most 64 per wave");
     constexpr int NG = H / QA;
+    const int HR = PAD ? D.H : H;  // slots
+    auto slot = [&](int c) { return PAD ? min(c, HR - 1) : c; };
     const int gw = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int n = b.cnt[cur];
@@ -165,7 +171,7 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
     // With one wave per token (QA == H) the Q|K|V rows are read once: non-temporal loads keep
     // them from displacing cached data.  With several, the waves of a token share K and V.
     constexpr bool NT = QA == H;
-    const float *base = b.qkv + (long)i * H * rowstride;
+    const float *base = b.qkv + (long)i * HR * rowstride;
 
     float part[QA][H];
 #pragma unroll
@@ -178,12 +184,12 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
 #pragma unroll
         for (int a = 0; a < QA; ++a)
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) q[a][v] = qkv_load<NT>(base + (long)(g * QA + a) * rowstride + off + v);
+            for (int v = 0; v < VEC; ++v) q[a][v] = qkv_load<NT>(base + (long)slot(g * QA + a) * rowstride + off + v);
 #pragma unroll
         for (int c = 0; c < H; ++c) {
             float kk[VEC];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) kk[v] = qkv_load<NT>(base + (long)c * rowstride + d + off + v);
+            for (int v = 0; v < VEC; ++v) kk[v] = qkv_load<NT>(base + (long)slot(c) * rowstride + d + off + v);
 #pragma unroll
             for (int a = 0; a < QA; ++a)
 #pragma unroll
@@ -226,11 +232,17 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
         const int gb = lane & ~(H - 1);
         float mx = -INFINITY;
 #pragma unroll
-        for (int c = 0; c < H; ++c) mx = fmaxf(mx, __shfl(sc, gb + c, 64));
+        for (int c = 0; c < H; ++c) {
+            const float v = __shfl(sc, gb + c, 64);
+            mx = !PAD || c < HR ? fmaxf(mx, v) : mx;
+        }
         const float ex = expf(sc - mx);
         float sum = 0.0f;
 #pragma unroll
-        for (int c = 0; c < H; ++c) sum += __shfl(ex, gb + c, 64);
+        for (int c = 0; c < H; ++c) {
+            const float v = __shfl(ex, gb + c, 64);
+            sum = !PAD || c < HR ? sum + v : sum;
+        }
         const float w_own = ex / sum;
         // every weight to every lane as a wave-uniform value (lane i holds index i)
 #pragma unroll
@@ -246,20 +258,20 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
                 float sc = wave_sum(part[a][c]) * scale;
                 if (D.flags & ADN_F_SCORE_CLAMP4) sc = fminf(fmaxf(sc, -4.0f), 4.0f);
                 e[c] = sc;
-                mx = fmaxf(mx, sc);
+                mx = !PAD || c < HR ? fmaxf(mx, sc) : mx;
             }
             float sum = 0.0f;
 #pragma unroll
             for (int c = 0; c < H; ++c) {
                 e[c] = expf(e[c] - mx);
-                sum += e[c];
+                sum = !PAD || c < HR ? sum + e[c] : sum;
             }
 #pragma unroll
             for (int c = 0; c < H; ++c) w[a * H + c] = e[c] / sum;
         }
     }
 
-    float *mixbase = b.mix + (long)i * H * d;
+    float *mixbase = b.mix + (long)i * HR * d;
     const float asc = b.mix_pre ? presplit_scale(b) : 1.0f;
     for (int off = lane * VEC; off < d; off += 64 * VEC) {
         float acc[QA][VEC];
@@ -271,15 +283,17 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
         for (int c = 0; c < H; ++c) {
             float vv[VEC];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) vv[v] = qkv_load<NT>(base + (long)c * rowstride + 2 * d + off + v);
+            for (int v = 0; v < VEC; ++v) vv[v] = qkv_load<NT>(base + (long)slot(c) * rowstride + 2 * d + off + v);
 #pragma unroll
             for (int a = 0; a < QA; ++a)
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) acc[a][v] = acc[a][v] + vv[v] * w[a * H + c];
+                for (int v = 0; v < VEC; ++v)
+                    acc[a][v] = !PAD || c < HR ? acc[a][v] + vv[v] * w[a * H + c] : acc[a][v];
         }
         if (b.mix_pre) {
 #pragma unroll
             for (int a = 0; a < QA; ++a) {
+                if (PAD && g * QA + a >= HR) break;
                 if constexpr (VEC == 4)  // lane pairs hold whole groups of 8 (off = 4 lane + 256 j)
                     store_presplit_pair(mixbase + (long)(g * QA + a) * d, off, acc[a], asc, lane);
                 else
@@ -287,88 +301,11 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
             }
         } else {
 #pragma unroll
-            for (int a = 0; a < QA; ++a)
+            for (int a = 0; a < QA; ++a) {
+                if (PAD && g * QA + a >= HR) break;
 #pragma unroll
                 for (int v = 0; v < VEC; ++v) mixbase[(long)(g * QA + a) * d + off + v] = acc[a][v];
-        }
-    }
-}
-
-// The same attention for any slot count H <= 16 (read at run time): one wave per (token, query
-// slot), the scores summed and the softmax formed as in k_attn's few-score path (the same
-// per-lane partial sums, one wave_sum per score, max and sum in key order).
-template <int VEC>
-__global__ __launch_bounds__(256) void k_attn_rt(Dims D, SolveBuffers b, int cur, int k) {
-    constexpr int HM = 16;
-    const int H = D.H;
-    const int gw = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int n = b.cnt[cur];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        b.cnt[cur ^ 1] = 0;
-        b.cnt_hist[k] += n;
-    }
-    const int i = gw / H, a = gw - (gw / H) * H;
-    if (i >= n) return;
-    const int d = D.d;
-    const long rowstride = 3L * d;
-    const float *base = b.qkv + (long)i * H * rowstride;
-    float part[HM];
-#pragma unroll
-    for (int c = 0; c < HM; ++c) part[c] = 0.0f;
-    for (int off = lane * VEC; off < d; off += 64 * VEC) {
-        float q[VEC];
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) q[v] = base[(long)a * rowstride + off + v];
-#pragma unroll
-        for (int c = 0; c < HM; ++c) {
-            if (c < H) {
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) part[c] += q[v] * base[(long)c * rowstride + d + off + v];
             }
-        }
-    }
-    const float scale = 1.0f / sqrtf((float)d);
-    float e[HM];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int c = 0; c < HM; ++c) {
-        if (c < H) {
-            float sc = wave_sum(part[c]) * scale;
-            if (D.flags & ADN_F_SCORE_CLAMP4) sc = fminf(fmaxf(sc, -4.0f), 4.0f);
-            e[c] = sc;
-            mx = fmaxf(mx, sc);
-        }
-    }
-    float sum = 0.0f;
-#pragma unroll
-    for (int c = 0; c < HM; ++c) {
-        if (c < H) {
-            e[c] = expf(e[c] - mx);
-            sum += e[c];
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < HM; ++c)
-        if (c < H) e[c] = e[c] / sum;
-    float *mixrow = b.mix + ((long)i * H + a) * d;
-    const float asc = b.mix_pre ? presplit_scale(b) : 1.0f;
-    for (int off = lane * VEC; off < d; off += 64 * VEC) {
-        float acc[VEC];
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < HM; ++c) {
-            if (c < H) {
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) acc[v] = acc[v] + base[(long)c * rowstride + 2 * d + off + v] * e[c];
-            }
-        }
-        if (b.mix_pre) {
-            store_presplit<VEC>(mixrow, off, acc, asc);
-        } else {
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) mixrow[off + v] = acc[v];
         }
     }
 }
@@ -603,8 +540,8 @@ __device__ void anderson_coeffs(int n, const float *g, float *beta) {
 // and one wave per slot, so that the slots' row updates run side by side instead of one after
 // another in a single wave.  Same arithmetic as k_update (the token residual is combined over
 // the slots in slot order).
-template <int E, bool PART>
-__global__ __launch_bounds__(1024) void k_update_tok(Dims D, SolveBuffers b, int cur, int k, int max_iters,
+template <int E, bool PART, int NTHR>
+__global__ __launch_bounds__(NTHR) void k_update_tok(Dims D, SolveBuffers b, int cur, int k, int max_iters,
                                                      float eps, const float *anchor, const float *norm_scale,
                                                      float beta) {
 #pragma clang fp contract(off)  // as in k_update
@@ -626,7 +563,8 @@ __global__ __launch_bounds__(1024) void k_update_tok(Dims D, SolveBuffers b, int
     float *hw = (b.h_out ? b.h_out : b.h) + ((long)t * H + s) * d;
     // every load (the norm scale too) before the first store of h: a load issued after stores
     // is waited for behind them (the vector-memory counter retires in issue order)
-    float cval[E], hold[E], gs[E];
+    constexpr int GC = E <= 16 ? E : 8;
+    float cval[E], hold[E], gs[GC];
     float ss = 0.0f;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -636,7 +574,7 @@ __global__ __launch_bounds__(1024) void k_update_tok(Dims D, SolveBuffers b, int
         const float c = as_ + (on ? an[idx] : 0.0f);
         cval[e] = c;
         hold[e] = on ? h[idx] : 0.0f;
-        gs[e] = on ? norm_scale[idx] : 0.0f;
+        if (GC == E) gs[e % GC] = on ? norm_scale[idx] : 0.0f;
         ss += excl ? as_ * as_ : c * c;
     }
     ss = wave_sum(ss);
@@ -645,7 +583,11 @@ __global__ __launch_bounds__(1024) void k_update_tok(Dims D, SolveBuffers b, int
     float r = 0.0f;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const float f = gs[e] * cval[e] / rms;
+        if (GC < E && e % GC == 0) {  // wide rows: the norm scale a group at a time (registers)
+#pragma unroll
+            for (int u = 0; u < GC; ++u) gs[u] = (!PART || e + u < er) ? norm_scale[lane + 64 * (e + u)] : 0.0f;
+        }
+        const float f = gs[e % GC] * cval[e] / rms;
         const float hn = f * beta + hold[e] * omb;
         if (!PART || e < er) {
             hw[lane + 64 * e] = hn;
@@ -684,8 +626,6 @@ __global__ __launch_bounds__(1024) void k_update_tok(Dims D, SolveBuffers b, int
 }
 
 constexpr int AND_NT = 256;
-// at most this many tokens in flight: the few-token kernel shapes (more waves per token)
-constexpr int SMALL_ROWS = 512;
 
 // The Anderson mix as one multiply-add chain per element, acc = fma(c_n-1, x_n-1, ... fma(c_0, x_0, 0)):
 // the fused update recomputes the previous iteration's mix with it, so both must round alike.
@@ -1295,17 +1235,28 @@ __global__ __launch_bounds__(AND_NT) void k_anderson_reg(Dims D, SolveBuffers b,
     }
 }
 
-template <int H, int QA>
+template <int H, int QA, bool PAD>
 void attn_dispatch_vec(const Dims &D, const SolveBuffers &b, int cur, int k, int ntok, hipStream_t st) {
     constexpr int NG = H / QA;
     const long waves = (long)ntok * NG;
     const dim3 grid((unsigned)((waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK));
     if (D.d % 256 == 0)
-        hipLaunchKernelGGL((k_attn<H, QA, 4>), grid, dim3(256), 0, st, D, b, cur, k);
+        hipLaunchKernelGGL((k_attn<H, QA, 4, PAD>), grid, dim3(256), 0, st, D, b, cur, k);
     else if (D.d % 128 == 0)
-        hipLaunchKernelGGL((k_attn<H, QA, 2>), grid, dim3(256), 0, st, D, b, cur, k);
+        hipLaunchKernelGGL((k_attn<H, QA, 2, PAD>), grid, dim3(256), 0, st, D, b, cur, k);
     else
-        hipLaunchKernelGGL((k_attn<H, QA, 1>), grid, dim3(256), 0, st, D, b, cur, k);
+        hipLaunchKernelGGL((k_attn<H, QA, 1, PAD>), grid, dim3(256), 0, st, D, b, cur, k);
+}
+
+// One wave per (token, query slot) for few tokens: the same scores, more waves; else QA query slots
+// per wave, which read K and V once per QA of them.
+template <int H, int QA>
+void attn_dispatch(const Dims &D, const SolveBuffers &b, int cur, int k, int ntok, bool few, hipStream_t st) {
+    const bool pad = D.H != H;
+    if (few)
+        pad ? attn_dispatch_vec<H, 1, true>(D, b, cur, k, ntok, st) : attn_dispatch_vec<H, 1, false>(D, b, cur, k, ntok, st);
+    else
+        pad ? attn_dispatch_vec<H, QA, true>(D, b, cur, k, ntok, st) : attn_dispatch_vec<H, QA, false>(D, b, cur, k, ntok, st);
 }
 
 }  // namespace
@@ -1318,35 +1269,21 @@ void launch_init(const Dims &D, const SolveBuffers &b, const float *x_src, const
 }
 
 void launch_attn(const Dims &D, const SolveBuffers &b, int cur, int k, int ntok, hipStream_t st) {
-    if (D.H & (D.H - 1)) {  // slot counts other than powers of two
-        const dim3 grid((unsigned)(((long)ntok * D.H + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK));
-        if (D.d % 256 == 0)
-            hipLaunchKernelGGL(k_attn_rt<4>, grid, dim3(256), 0, st, D, b, cur, k);
-        else if (D.d % 128 == 0)
-            hipLaunchKernelGGL(k_attn_rt<2>, grid, dim3(256), 0, st, D, b, cur, k);
-        else
-            hipLaunchKernelGGL(k_attn_rt<1>, grid, dim3(256), 0, st, D, b, cur, k);
-        return;
-    }
-    if (ntok <= SMALL_ROWS) {  // one wave per (token, query slot): the same scores, more waves
-        switch (D.H) {
-            case 1: attn_dispatch_vec<1, 1>(D, b, cur, k, ntok, st); break;
-            case 2: attn_dispatch_vec<2, 1>(D, b, cur, k, ntok, st); break;
-            case 4: attn_dispatch_vec<4, 1>(D, b, cur, k, ntok, st); break;
-            case 8: attn_dispatch_vec<8, 1>(D, b, cur, k, ntok, st); break;
-            case 16: attn_dispatch_vec<16, 1>(D, b, cur, k, ntok, st); break;
-            default: break;
-        }
-        return;
-    }
-    switch (D.H) {
-        case 1: attn_dispatch_vec<1, 1>(D, b, cur, k, ntok, st); break;
-        case 2: attn_dispatch_vec<2, 2>(D, b, cur, k, ntok, st); break;
-        case 4: attn_dispatch_vec<4, 4>(D, b, cur, k, ntok, st); break;
-        case 8: attn_dispatch_vec<8, 8>(D, b, cur, k, ntok, st); break;
-        case 16: attn_dispatch_vec<16, 4>(D, b, cur, k, ntok, st); break;
-        default: break;  // other slot counts take k_attn_rt
-    }
+    // a wave per query slot, which reads all K and V rows of its token, while the tokens are few:
+    // us against QA query slots per wave, 8 slots of 512: 513 tokens 13.7 / 18.5, 1024 21.6 / 22.4,
+    // 2048 37.4 / 29.8; 16 slots of 1024: 256 tokens 34 / 47, 512 63 / 53; 12 slots of 512 (padded):
+    // 300 tokens 47, 512 tokens at QA = 4 30
+    const bool few = ntok <= (D.H == 16 ? 256 : D.H > 8 ? 128 : 1024);
+    if (D.H == 1)
+        attn_dispatch_vec<1, 1, false>(D, b, cur, k, ntok, st);
+    else if (D.H == 2)
+        few ? attn_dispatch_vec<2, 1, false>(D, b, cur, k, ntok, st) : attn_dispatch_vec<2, 2, false>(D, b, cur, k, ntok, st);
+    else if (D.H <= 4)
+        attn_dispatch<4, 4>(D, b, cur, k, ntok, few, st);
+    else if (D.H <= 8)
+        attn_dispatch<8, 8>(D, b, cur, k, ntok, few, st);
+    else
+        attn_dispatch<16, 4>(D, b, cur, k, ntok, few, st);
 }
 
 // k_update for d = 64 E: the slot count as a template argument (1, 2, 4, 8, 16) up to d = 1024
@@ -1366,7 +1303,12 @@ void launch_update_e(const Dims &D, const SolveBuffers &b, int cur, int k, int m
             case 2: hipLaunchKernelGGL((k_update<E, 2, false, false>), grid, blk, 0, st, ADN_UPD_ARGS); return;
             case 4: hipLaunchKernelGGL((k_update<E, 4, false, false>), grid, blk, 0, st, ADN_UPD_ARGS); return;
             case 8: hipLaunchKernelGGL((k_update<E, 8, false, false>), grid, blk, 0, st, ADN_UPD_ARGS); return;
-            case 16: hipLaunchKernelGGL((k_update<E, 16, false, false>), grid, blk, 0, st, ADN_UPD_ARGS); return;
+            case 16:
+                if constexpr (E <= 8) {  // 16 slots of 1024, unrolled, spill: 162 us at 531 tokens
+                    hipLaunchKernelGGL((k_update<E, 16, false, false>), grid, blk, 0, st, ADN_UPD_ARGS);
+                    return;
+                }
+                break;
             default: break;
         }
     }
@@ -1376,12 +1318,30 @@ void launch_update_e(const Dims &D, const SolveBuffers &b, int cur, int k, int m
 
 void launch_update(const Dims &D, const SolveBuffers &b, int cur, int k, int max_iters, float eps, int ntok,
                    const float *anchor, const float *norm_scale, float beta, hipStream_t st) {
-    if (ntok <= SMALL_ROWS) {
+    // a wave per slot until the waves of k_update, one per token walking its slots, fill the chip as
+    // well: us of the two at d = 512, H = 8: 513 tokens 13.9 / 18.6, 1024 21.4 / 21.1, 2048 34.6 / 28.6;
+    // d = 1024, H = 16: 513 tokens 33 / 54, 1500 86 / 84; H = 3: 512 tokens 11.8 / 12.0.  Rows beyond
+    // 1024 hold twice the registers: 512 tokens of 8 x 2048 39 / 54, 900 64 / 60; over 8 slots a block
+    // leaves 128 registers per lane and spills: 128 tokens of 16 x 2048 68 / 90, 300 126 / 94.
+    const int tok_rows = D.d <= 1024 ? 128 * D.H : D.H <= 8 ? 64 * D.H : 12 * D.H;
+    if (ntok <= tok_rows) {
         const dim3 tgrid((unsigned)ntok), tblk(64 * D.H);
         const size_t lds = b.pool ? (size_t)D.H * D.d * sizeof(float) : 0;
         dispatch_width(D.d, [&](auto Ec, auto Pc) {
-            hipLaunchKernelGGL((k_update_tok<decltype(Ec)::value, decltype(Pc)::value>), tgrid, tblk, lds, st, D, b,
-                               cur, k, max_iters, eps, anchor, norm_scale, beta);
+            constexpr int E = decltype(Ec)::value;
+            constexpr bool P = decltype(Pc)::value;
+#define ADN_TOK_ARGS tgrid, tblk, lds, st, D, b, cur, k, max_iters, eps, anchor, norm_scale, beta
+            if constexpr (E > 16) {  // wide rows: the registers that the block's size leaves
+                if (D.H <= 4)
+                    hipLaunchKernelGGL((k_update_tok<E, P, 256>), ADN_TOK_ARGS);
+                else if (D.H <= 8)
+                    hipLaunchKernelGGL((k_update_tok<E, P, 512>), ADN_TOK_ARGS);
+                else
+                    hipLaunchKernelGGL((k_update_tok<E, P, 1024>), ADN_TOK_ARGS);
+            } else {
+                hipLaunchKernelGGL((k_update_tok<E, P, 1024>), ADN_TOK_ARGS);
+            }
+#undef ADN_TOK_ARGS
         });
         return;
     }

@@ -44,3 +44,24 @@ def test_tiles_match_oracle(shape, flags):
     # the fused arg-max is the last-max of the stored logits
     lg = got["logits"].reshape(-1, V)
     assert np.array_equal(got["argmax"].ravel(), V - 1 - np.argmax(lg[:, ::-1], axis=1))
+
+
+# tokens on both sides of the attention's and the update's few-token limits, padded slot counts and
+# rows beyond 1024 floats
+@pytest.mark.parametrize("d,H,n", [(64, 3, 385), (128, 5, 641), (64, 8, 1024), (64, 8, 1025), (192, 12, 128),
+                                   (128, 12, 129), (64, 16, 256), (64, 16, 257), (320, 6, 1030), (1024, 16, 40),
+                                   (1536, 3, 70), (2048, 2, 129), (2048, 9, 12)])
+def test_token_limits_match_oracle(d, H, n):
+    from oracle import pyoracle
+    mc = synth.ModelConfig(d=d, H=H, V=33, N=1, max_iters=2, eps=0.0)
+    w = synth.make_token_sensitive_weights(mc)
+    toks = synth.make_tokens("uniform", 1, n, mc.V, seed=1)
+    be = GpuDeqBackend(mc, 1, n)
+    be.upload_weights(w)
+    got = be.forward(toks, want=("h_star", "iters"))
+    be.close()
+    # the tokens of one id are alike: every row against the oracle's solve of its id
+    ids, inv = np.unique(toks[0], return_inverse=True)
+    ref = pyoracle.Oracle(mc, w).forward(ids[None].astype(np.int32), nthreads=8, want_scan=False)
+    np.testing.assert_allclose(got["h_star"][0], ref["h_star"][0][inv], rtol=RTOL, atol=ATOL)
+    assert (got["iters"] == 2).all()
