@@ -858,27 +858,30 @@ void launch_skinny(const GemmParams &p, int kw, hipStream_t st) {
     }
 }
 
-// Tiles of a GEMM below the 256x256 range: the configuration with the least a + b * (its blocks),
-// in us for K = 512, a fit to measured back-to-back launches of 8-slot products at 5 to 1000 rows
-// and N = 64 to 1536 (other K scale all of them alike).  a is the latency of one block's chain,
-// b the chip's time per block once the blocks outnumber the CUs:
-//   32x32   K-sliced over 8 waves   256 blocks  5.2 us,  768 blocks 10.0
-//   32x64   K-sliced over 4 waves   256 blocks  7.0 us,  768 blocks 14.1
-//   64x64   K-sliced over 4 waves   256 blocks 10.4 us,  768 blocks 23.6
-//   64x128  ring, waves of 32x64    256 blocks 14.1 us,  864 blocks 34.2
-//   128x128 ring, waves of 32x128   256 blocks 19.8 us,  768 blocks 44.2
-enum TilePick { TP_KS32, TP_KS32X64, TP_KS64, TP_R64X128, TP_R128 };
+// Tiles of a product of M rows: the configuration with the least a + b * (its blocks / 256), for the
+// ring kernels rounded up to whole rounds of one block per CU (the K-sliced blocks are small enough
+// to fill in); us for K = 512 (other K scale all of them alike), fitted to back-to-back launches of 8- and 16-slot products at 5 to 8192 rows, N = 64 to 3072:
+//   32x32   K-sliced over 8 waves   256 blocks  5.2 us,  768 blocks  10.0, 1536 blocks  18.6
+//   32x64   K-sliced over 4 waves   256 blocks  7.0 us,  768 blocks  14.1, 1536 blocks  24.4
+//   64x64   K-sliced over 4 waves   256 blocks 10.4 us,  768 blocks  23.6, 1024 blocks  30.1
+//   64x128  ring, waves of 32x64    192 blocks 12.1 us,  672 blocks  26.0, 1248 blocks  42.7
+//   64x256  ring, waves of 32x128   192 blocks 17.3 us,  432 blocks  27.7, 1008 blocks  56.9
+//   128x128 ring, waves of 32x128   256 blocks 18.7 us,  768 blocks  43.0, 3072 blocks 163
+//   256x256 ring, persistent        192 blocks 47.7 us,  768 blocks 157,   1536 blocks 300
+// The 256x256 blocks do the least work per value, and lose where their last round is nearly empty:
+// 1500 rows of Q|K|V (288 blocks) 85 us against 66 on 128x128 blocks, W_o 34 against 22.
+enum TilePick { TP_KS32, TP_KS32X64, TP_KS64, TP_R64X128, TP_R64X256, TP_R128, TP_R256 };
 TilePick pick_tiles(int M, int N, int S) {
     static const struct {
         int bm, bn;
         float a, b;
-    } cf[] = {{32, 32, 3.0f, 0.0101f}, {32, 64, 4.0f, 0.0135f}, {64, 64, 5.0f, 0.0255f}, {64, 128, 10.0f, 0.0285f},
-              {128, 128, 13.0f, 0.041f}};
+    } cf[] = {{32, 32, 3.0f, 2.6f}, {32, 64, 4.0f, 3.5f}, {64, 64, 5.0f, 6.5f},     {64, 128, 3.0f, 8.7f},
+              {64, 256, 5.5f, 13.0f}, {128, 128, 5.0f, 13.0f}, {256, 256, 3.0f, 46.0f}};
     int best = 0;
     float least = INFINITY;
-    for (int i = 0; i < 5; ++i) {
-        const float n = (float)((M + cf[i].bm - 1) / cf[i].bm) * (float)((N + cf[i].bn - 1) / cf[i].bn) * (float)S;
-        const float t = cf[i].a + cf[i].b * n;
+    for (int i = 0; i < 7; ++i) {
+        const long n = (long)((M + cf[i].bm - 1) / cf[i].bm) * ((N + cf[i].bn - 1) / cf[i].bn) * S;
+        const float t = cf[i].a + cf[i].b * (i < TP_R64X128 ? (float)n / 256.0f : (float)((n + 255) / 256));
         if (t < least) {
             least = t;
             best = i;
@@ -887,37 +890,58 @@ TilePick pick_tiles(int M, int N, int S) {
     return (TilePick)best;
 }
 
-int tiles(const GemmParams &p, int bm, int bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.S; }
-
-// The LM head below the 256x256 range, its blocks holding whole arg-max partials (128 columns):
-// 64x256 blocks of 32x128 waves, each A fragment split once per four column tiles (V = 50257,
-// K = 512: 64 rows 38.5 -> 23 us, 128 rows 38 -> 33, 531 rows 168 -> 138, 900 rows 263 -> 231
-// against the 128x128 blocks of 64x64 waves used before); a head too narrow to fill the chip takes
-// 64x128 blocks of 32x64 waves (V = 65, K = 192: 15.8 -> 9.8 us).
-template <typename T, int TERMS>
-void launch_lm_mid(const GemmParams &p, hipStream_t st) {
-    const int wide = tiles(p, 64, 256);
-    if (wide >= 64)
-        hipLaunchKernelGGL((k_gemm_split<ROLE_LMHEAD, T, TERMS, 1, 4, 2, 2, 4>), dim3(wide), dim3(256), 0, st, p);
-    else
-        hipLaunchKernelGGL((k_gemm_split<ROLE_LMHEAD, T, TERMS, 1, 2, 2, 2, 4>), dim3(tiles(p, 64, 128)), dim3(256), 0,
-                           st, p);
+// The LM head's blocks hold whole arg-max partials (128 columns): 64x256 up to 64 rows, 128x128
+// above, both of 32x128 waves, or 256x256 (costs as above); a head too narrow to fill the chip takes
+// 64x128 blocks.  V = 50257, K = 512, A pre-split: 64 rows 38.5 us (128x128 blocks of 64x64 waves) ->
+// 23, 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8 us.
+TilePick pick_lm_tiles(int M, int V) {
+    const int nv = (V + 127) / 128;
+    if ((M + 127) / 128 * nv < 64) return TP_R64X128;
+    if (M <= 64) return TP_R64X256;
+    const int r128 = ((M + 127) / 128 * nv + 255) / 256, r256 = ((M + 255) / 256 * ((V + 255) / 256) + 255) / 256;
+    return 5.0f + 13.0f * r128 < 3.0f + 46.0f * r256 ? TP_R128 : TP_R256;
 }
 
-// Tile configurations (WTM, WTN, WGM, WGN, STAGES): GEMMs with M >= 1024 and N >= 512 use
-// 256x256 blocks of 8 waves (one workgroup per CU, 128 KB of LDS ring), persistent (one resident
-// workgroup per CU walking its share of tiles, the next tile's first slices loaded during the
-// epilogue); the rest take what pick_tiles says, a workgroup per tile.
+int tiles(const GemmParams &p, int bm, int bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.S; }
+
+// The ring kernel on the picked blocks (template order WTM, WTN, WGM, WGN, STAGES); PRE: A pre-split
+// by its producer.  The 256x256 blocks run persistent (8 waves, one resident workgroup per CU
+// walking its share of tiles, the next tile's first slices loaded during the epilogue), the smaller
+// ones a workgroup per tile, whose short k loops would otherwise wait on the previous tile's stores.
+template <int ROLE, typename T, int TERMS, bool PRE>
+void launch_ring(const GemmParams &p, TilePick tp, hipStream_t st) {
+    switch (tp) {
+        case TP_R64X128:
+            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 2, 2, 2, 4, PRE>), dim3(tiles(p, 64, 128)), dim3(256), 0, st, p);
+            break;
+        case TP_R64X256:
+            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 2, 2, 4, PRE>), dim3(tiles(p, 64, 256)), dim3(256), 0, st, p);
+            break;
+        case TP_R128:
+            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
+            break;
+        default: {
+            const int grid = ring_grid(tiles(p, 256, 256), 1);
+            if constexpr (ROLE == ROLE_QKV)
+                // waves of 32 x 256 (8 down the block): each A row block is split by one wave only
+                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 8, 8, 1, 4, PRE>), dim3(grid), dim3(512), 0, st, p);
+            else
+                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4, PRE>), dim3(grid), dim3(512), 0, st, p);
+        }
+    }
+}
+
 template <int ROLE, typename T, int TERMS>
 void launch_cfg(const GemmParams &p, hipStream_t st) {
     if (p.M <= 0 || p.N <= 0 || p.S <= 0) return;
+    constexpr bool F16 = std::is_same<T, _Float16>::value;
     // K split over the waves of the few-row kernel, about two 64-K steps per wave (every K is a
     // multiple of 64), each wave's K range whole 64-K steps
     const int steps = p.K / 64;
     int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
     while (steps % kw) kw >>= 1;
     if constexpr (ROLE == ROLE_LMHEAD) {
-        if (p.M <= 32) {
+        if (p.M <= LM_SKINNY_ROWS) {
             // skinny LM head (a decode step): 128-column blocks, the arg-max partials' width; at
             // a few rows 64-column blocks with partials per 64 columns (twice the workgroups on
             // the weight stream)
@@ -927,63 +951,48 @@ void launch_cfg(const GemmParams &p, hipStream_t st) {
                 launch_skinny<ROLE, T, TERMS, 4>(p, kw, st);
             return;
         }
-    } else if (p.M <= ATTN_FUSE_ROWS) {
-        // a few rows: one 32-column tile per wave (decode Q|K|V at one row against two tiles:
-        // 248 -> 238 us per token).  The forms with a fused stage and the plain one are the same
-        // product bit for bit.
-        if constexpr (ROLE == ROLE_WO) {
-            if (p.attn_qkv) {  // the attention formed in the kernel
-                launch_skinny<ROLE, T, TERMS, 1, true>(p, kw, st);
-                return;
-            }
-        }
-        if constexpr (ROLE == ROLE_QKV) {
-            if (p.upd_o) {  // the previous iteration's update formed in the kernel
-                launch_skinny<ROLE, T, TERMS, 1, false, true>(p, kw, st);
-                return;
-            }
-        }
-        launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
+        launch_ring<ROLE, T, TERMS, F16>(p, pick_lm_tiles(p.M, p.N), st);  // fp16: gemm_lm_presplit
         return;
-    }
-    if (p.N >= 512 && p.M >= 1024) {  // the configuration gemm_presplit_ok names
-        const int total = tiles(p, 256, 256);
-        // the roles whose A a producer writes pre-split (the slot mix, the LM head's normalised row)
-        if constexpr (std::is_same<T, _Float16>::value && TERMS == 3 && (ROLE == ROLE_WO || ROLE == ROLE_LMHEAD)) {
-            if (p.a_pre) {
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4, true>), dim3(ring_grid(total, 1)),
-                                   dim3(512), 0, st, p);
-                return;
-            }
-        }
-        if constexpr (ROLE == ROLE_QKV)
-            // waves of 32 x 256 (8 down the block): each A row block is split by one wave only
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 8, 8, 1, 4>), dim3(ring_grid(total, 1)), dim3(512), 0, st,
-                               p);
-        else
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4>), dim3(ring_grid(total, 1)), dim3(512), 0, st,
-                               p);
-        return;
-    }
-    if constexpr (ROLE == ROLE_LMHEAD) {
-        launch_lm_mid<T, TERMS>(p, st);
     } else {
+        if (p.M <= ATTN_FUSE_ROWS) {
+            // a few rows: one 32-column tile per wave (decode Q|K|V at one row against two tiles:
+            // 248 -> 238 us per token).  The forms with a fused stage and the plain one are the same
+            // product bit for bit.
+            if constexpr (ROLE == ROLE_WO) {
+                if (p.attn_qkv) {  // the attention formed in the kernel
+                    launch_skinny<ROLE, T, TERMS, 1, true>(p, kw, st);
+                    return;
+                }
+            }
+            if constexpr (ROLE == ROLE_QKV) {
+                if (p.upd_o) {  // the previous iteration's update formed in the kernel
+                    launch_skinny<ROLE, T, TERMS, 1, false, true>(p, kw, st);
+                    return;
+                }
+            }
+            launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
+            return;
+        }
         if (p.N <= 64 && p.M >= 1024) {
             // narrow outputs (the carrier's projections, r + 2N = 64 columns): 128 x 64 blocks of two
             // 64 x 64 waves, no zero-padded half tile
             hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 1, 4>), dim3(tiles(p, 128, 64)), dim3(128), 0, st, p);
             return;
         }
-        switch (pick_tiles(p.M, p.N, p.S)) {
-            case TP_KS32: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 8, 1, 1>), dim3(tiles(p, 32, 32)), dim3(512), 0, st, p); break;
-            case TP_KS32X64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 1, 2>), dim3(tiles(p, 32, 64)), dim3(256), 0, st, p); break;
-            case TP_KS64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 2, 2>), dim3(tiles(p, 64, 64)), dim3(256), 0, st, p); break;
-            case TP_R64X128:
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 2, 2, 2, 4>), dim3(tiles(p, 64, 128)), dim3(256), 0, st, p);
-                break;
-            default:
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
+        const TilePick tp = pick_tiles(p.M, p.N, p.S);
+        switch (tp) {
+            case TP_KS32: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 8, 1, 1>), dim3(tiles(p, 32, 32)), dim3(512), 0, st, p); return;
+            case TP_KS32X64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 1, 2>), dim3(tiles(p, 32, 64)), dim3(256), 0, st, p); return;
+            case TP_KS64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 2, 2>), dim3(tiles(p, 64, 64)), dim3(256), 0, st, p); return;
+            default: break;
         }
+        if constexpr (F16 && ROLE == ROLE_WO) {
+            if (p.a_pre) {  // gemm_wo_presplit
+                launch_ring<ROLE, T, TERMS, true>(p, tp, st);
+                return;
+            }
+        }
+        launch_ring<ROLE, T, TERMS, false>(p, tp, st);
     }
 }
 
@@ -1009,7 +1018,11 @@ void launch_gemm_split(const GemmParams &p, hipStream_t st) {
     }
 }
 
-bool gemm_presplit_ok(int prec, int M, int N) { return prec == PREC_F16X3 && M >= 1024 && N >= 512; }
+bool gemm_wo_presplit(int prec, int M, int N, int S) {
+    return prec == PREC_F16X3 && M > ATTN_FUSE_ROWS && !(N <= 64 && M >= 1024) && pick_tiles(M, N, S) >= TP_R64X128;
+}
+
+bool gemm_lm_presplit(int prec, int M) { return prec == PREC_F16X3 && M > LM_SKINNY_ROWS; }
 
 int gemm_lm_partial_cols(int prec, int M, int K) {
     return (prec != PREC_FP32 && M <= ATTN_FUSE_ROWS && K % 64 == 0) ? 64 : GEMM_BN;

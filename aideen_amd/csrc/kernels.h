@@ -77,8 +77,8 @@ struct GemmParams {
     const unsigned *a_absmax;
     float a_headroom;
     // A given instead as fp16 hi/lo halves split by its producer with the kernel's own A scale
-    // (k_gemm_split's pre-split layout); W_o and the LM head, for the shapes gemm_presplit_ok
-    // names; null = none
+    // (k_gemm_split's pre-split layout); W_o and the LM head, for the shapes gemm_wo_presplit and
+    // gemm_lm_presplit name; null = none
     const float *a_pre;
     // W_o on at most ATTN_FUSE_ROWS rows (the skinny kernel, split arithmetic): with attn_qkv set
     // the A operand (the attention mix of slot s) is formed in the kernel from the compact
@@ -103,12 +103,14 @@ struct GemmParams {
     int upd_excl;              // ADN_F_RMS_EXCL_ANCHOR
 };
 constexpr int ATTN_FUSE_ROWS = 4;
+constexpr int LM_SKINNY_ROWS = 32;  // the LM head's few-row kernel
 constexpr int GEMM_BN = 128;
 void launch_gemm(const GemmParams &p, hipStream_t st);
 void launch_gemm_split(const GemmParams &p, hipStream_t st);
-// Whether a split GEMM of this shape reads a pre-split A operand (GemmParams::a_pre): fp16
-// halves and the 256x256 persistent tiles (M >= 1024, N >= 512).
-bool gemm_presplit_ok(int prec, int M, int N);
+// Whether the product reads its A operand pre-split (GemmParams::a_pre): fp16 halves, W_o of M rows
+// and S slots on the ring kernel's tiles, the LM head beyond the skinny kernel's rows.
+bool gemm_wo_presplit(int prec, int M, int N, int S);
+bool gemm_lm_presplit(int prec, int M);
 // Whether W_o on at most M rows runs with the attention formed in its kernel (GemmParams::attn_qkv):
 // the skinny split-arithmetic kernel, M <= ATTN_FUSE_ROWS, K a multiple of 64, at most 16 slots.
 bool gemm_attn_fusable(int prec, int M, int K, int S);

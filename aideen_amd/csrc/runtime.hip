@@ -375,9 +375,9 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
     // Anderson depths 1 and 2 never mix (n_res = min(k, m - 1) < 2), so they run as plain Picard
     // (no ring of iterates)
     const int m = c->cfg.anderson_m >= 3 ? c->cfg.anderson_m : 0;
-    // W_o on the 256x256 fp16-split tiles reads its A (mix) pre-split: the attention writes the
+    // W_o on the fp16-split ring tiles reads its A (mix) pre-split: the attention writes the
     // halves, in mix's memory, with the scale the GEMM derives from the h bound (set_range below)
-    const bool wo_pre = gemm_presplit_ok(c->prec, rows, d);
+    const bool wo_pre = gemm_wo_presplit(c->prec, rows, d, H);
     SolveBuffers ba = b;
     if (wo_pre) {
         ba.mix_pre = b.mix;
@@ -567,9 +567,9 @@ bool enqueue_head(adn_ctx *c, const adn_outputs &o, const SolveBuffers &b, int n
     hipStream_t st = c->stream;
     const bool want_logits = o.logits || o.argmax;
     const bool pool = o.pooled || want_logits;
-    // the LM head on the 256x256 fp16-split tiles reads its A pre-split, written so by the pool
+    // the LM head beyond a few rows, on fp16 halves, reads its A pre-split, written so by the pool
     // kernel with the head's A scale
-    const bool lm_pre = want_logits && gemm_presplit_ok(c->prec, ntok, D.V);
+    const bool lm_pre = want_logits && gemm_lm_presplit(c->prec, ntok);
     if (pool && !pool_done) {
         Span sp(prof, ADN_STAGE_POOL, -1, st);
         launch_pool_norm(D, b.h, ntok, c->lm_g, o.pooled, want_logits ? c->pnorm : nullptr,
@@ -691,7 +691,7 @@ void enqueue_forward(adn_ctx *c, const adn_run &r, const adn_outputs &o, Prof *p
     pr.pool_out = o.pooled;
     pr.pool_norm = want_logits ? c->pnorm : nullptr;
     pr.pool_g = c->lm_g;
-    const bool pool_ok = (want_logits || o.pooled) && !scan && !(want_logits && gemm_presplit_ok(c->prec, ntok, c->D.V));
+    const bool pool_ok = (want_logits || o.pooled) && !scan && !(want_logits && gemm_lm_presplit(c->prec, ntok));
     const bool pooled = enqueue_iterations(c, r, b, ntok, ntok, prof, pool_ok ? &pr : nullptr);
     const bool prep_done = enqueue_head(c, o, b, ntok, prof, scan, ds ? ds->app : nullptr, pooled);
     enqueue_scan(c, r, o, b, prof, prep_done);
