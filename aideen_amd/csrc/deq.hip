@@ -158,10 +158,10 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
     auto slot = [&](int c) { return PAD ? min(c, HR - 1) : c; };
     const int gw = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int n = b.cnt[cur];
+    const int n = b.all_rows ? b.all_rows : b.cnt[cur];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         // the update kernel of this iteration appends survivors to the other list
-        b.cnt[cur ^ 1] = 0;
+        if (!b.all_rows) b.cnt[cur ^ 1] = 0;
         b.cnt_hist[k] += n;  // summed over the positions of a memory-coupled forward
     }
     const int i = gw / NG, g = gw - (gw / NG) * NG;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void k_update(Dims D, SolveBuffers b, int cur,
     __shared__ int keep_s[WAVES_PER_BLOCK];
     __shared__ int tok_s[WAVES_PER_BLOCK];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int n = b.cnt[cur];
+    const int n = b.all_rows ? b.all_rows : b.cnt[cur];
     if (blockIdx.x * WAVES_PER_BLOCK >= n) return;
     const int i = blockIdx.x * WAVES_PER_BLOCK + wave;
     const int H = HT > 0 ? HT : D.H;
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(256) void k_update(Dims D, SolveBuffers b, int cur,
     bool keep = false;
     int t = -1;
     if (i < n) {
-        t = b.act[cur][i];
+        t = b.ident ? i : b.act[cur][i];
         float g[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) g[e] = (!PART || e < er) ? norm_scale[lane + 64 * e] : 0.0f;
@@ -449,13 +449,15 @@ __global__ __launch_bounds__(256) void k_update(Dims D, SolveBuffers b, int cur,
             }
         }
         if (rmode == 1) rtok = nan_to_inf(sqrtf(rtok));
-        const int ex = token_exit(rtok, eps, k, max_iters, b.rprev ? b.rprev + t : nullptr, lane == 0);
+        const int ex = b.all_rows ? (k + 1 >= max_iters ? 2 : 0)
+                                  : token_exit(rtok, eps, k, max_iters, b.rprev ? b.rprev + t : nullptr, lane == 0);
         if (ex && lane == 0) {
             b.iters[t] = k + 1;
             if (b.conv) b.conv[t] = ex == 1;
         }
         keep = !ex || (ex == 2 && b.cap_mix);
     }
+    if (b.all_rows) return;
     if (lane == 0) {
         keep_s[wave] = keep;
         tok_s[wave] = t;
@@ -548,13 +550,14 @@ __global__ __launch_bounds__(NTHR) void k_update_tok(Dims D, SolveBuffers b, int
     __shared__ float rs[16];
     extern __shared__ float hl[];  // [H][d] the new rows, with b.pool
     const int i = blockIdx.x;
-    if (i >= b.cnt[cur]) return;
+    const int n = b.all_rows ? b.all_rows : b.cnt[cur];
+    const int t = b.ident ? i : b.act[cur][i];  // past the count: not used
+    if (i >= n) return;
     const int s = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int H = D.H;
     const int d = PART ? D.d : 64 * E, er = PART ? D.d / 64 : E;  // chunks e >= er are outside the row
     const bool excl = (D.flags & ADN_F_RMS_EXCL_ANCHOR) != 0;
     const int rmode = (D.flags & ADN_F_RESID_L2) ? 1 : (D.flags & ADN_F_RESID_RELRMS) ? 2 : 0;
-    const int t = b.act[cur][i];
     const float *o = b.o + ((long)i * H + s) * d;
     const float *sg = b.signal + ((long)t * H + s) * d;
     const float *an = anchor + (long)s * d;
@@ -597,10 +600,19 @@ __global__ __launch_bounds__(NTHR) void k_update_tok(Dims D, SolveBuffers b, int
         const float df = hn - hold[e];
         r = rmode ? r + df * df : fmaxf(r, nan_to_inf(fabsf(df)));
     }
-    r = rmode ? wave_sum(r) : wave_max(r);
-    if (lane == 0) rs[s] = slot_resid(rmode, r, rms, d);
-    __syncthreads();
-    if (threadIdx.x == 0) {
+    if (b.all_rows) {
+        if (threadIdx.x == 0 && k + 1 >= max_iters) {
+            b.iters[t] = k + 1;
+            if (b.conv) b.conv[t] = 0;
+        }
+        if (!b.pool) return;
+        __syncthreads();
+    } else {
+        r = rmode ? wave_sum(r) : wave_max(r);
+        if (lane == 0) rs[s] = slot_resid(rmode, r, rms, d);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && !b.all_rows) {
         float rtok = 0.0f;
         for (int q = 0; q < H; ++q) rtok = combine_resid(rmode, rtok, rs[q]);
         if (rmode == 1) rtok = nan_to_inf(sqrtf(rtok));

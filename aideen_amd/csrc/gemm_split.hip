@@ -414,8 +414,8 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_skinny(GemmParams p) {
     map_block(blockIdx.x, nN * p.S, 1, nN, s, mt, nt);
     if constexpr (ATTN) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {  // the attention kernel's bookkeeping
-            const int n = *p.m_count;
-            *p.attn_cnt_next = 0;  // the update of this iteration appends survivors there
+            const int n = p.m_count ? *p.m_count : p.M;
+            if (p.attn_cnt_next) *p.attn_cnt_next = 0;  // the update of this iteration appends survivors there
             *p.attn_cnt_hist += n;
         }
     }
@@ -676,14 +676,21 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 4 : (WTM == 2 ? 2 : 4)) void k_g
     constexpr int BMt = 32 * WTM, BNt = 32 * WTN;
     __shared__ float red[KW][NE][64];
     const int nM = (p.M + BMt - 1) / BMt, nN = (p.N + BNt - 1) / BNt;
-    const int M = p.m_count ? min(*p.m_count, p.M) : p.M;
     int s, mt, nt;
     map_block(blockIdx.x, nM * nN * p.S, nM, nN, s, mt, nt);
     const int m0 = mt * BMt, n0 = nt * BNt;
-    if (m0 >= M) return;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int q = lane & 31, g = lane >> 5;
+    // the row indices are loaded beside the count, not behind it (entries past it are not used)
+    int ridx[WTM];
+#pragma unroll
+    for (int i = 0; i < WTM; ++i) {
+        const int m = min(m0 + 32 * i + q, p.M - 1);
+        ridx[i] = p.a_idx ? p.a_idx[m] : m;
+    }
+    const int M = p.m_count ? min(*p.m_count, p.M) : p.M;
+    if (m0 >= M) return;
     const int steps = p.K / BK;
     const int sb = wave * steps / KW, se = (wave + 1) * steps / KW;  // this wave's steps
     // rows past M read row 0, column groups past N group 0 (their outputs are not stored)
@@ -693,7 +700,7 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 4 : (WTM == 2 ? 2 : 4)) void k_g
         const int m = m0 + 32 * i + q;
         long ar = 0;
         if (m < M) {
-            ar = p.a_idx ? (long)p.a_idx[m] : (long)m;
+            ar = ridx[i];
             if (p.a_idx && (ar < 0 || ar >= p.a_idx_max)) {
                 if (p.err) atomicOr(p.err, ADN_DEVERR_TOKEN);
                 ar = 0;

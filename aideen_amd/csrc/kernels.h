@@ -86,7 +86,7 @@ struct GemmParams {
     // that kernel's bookkeeping (attn_cnt_next = 0, attn_cnt_hist += the active count)
     const float *attn_qkv;
     int attn_clamp;            // ADN_F_SCORE_CLAMP4
-    int32_t *attn_cnt_next;
+    int32_t *attn_cnt_next;    // null where the list serves every iteration (SolveBuffers::all_rows)
     int32_t *attn_cnt_hist;
     // Q|K|V on at most ATTN_FUSE_ROWS rows (the skinny kernel, split arithmetic) when no token can
     // exit early: with upd_o set the kernel first applies the previous iteration's damped update
@@ -172,6 +172,11 @@ struct SolveBuffers {
     float *pool_out;
     float *pool_norm;
     const float *pool_g;
+    // > 0: no token can exit before the last iteration (a tolerance of zero or less, no plateau
+    // exit), so list 0 with this many rows serves every iteration: its count is not read, nothing
+    // is appended and no residual is formed.  ident: list 0 is 0, 1, 2, ... and is not read either
+    int all_rows;
+    int ident;
     // [ntok][4] the coefficients of each token's last Anderson mix (launch_update_mix), or null
     float *mix_coef;
 };

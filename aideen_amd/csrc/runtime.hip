@@ -367,7 +367,7 @@ void enqueue_signal_init(adn_ctx *c, const adn_run &r, const SolveBuffers &b, in
 // active, token indices are < ntok (the row stride of h, signal and the Anderson ring).
 // pool: the head's pool outputs (SolveBuffers::pool_*), formed by the last update where it can
 // (a fixed-iteration solve whose rows fit in LDS); returns whether it did.
-bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int rows, int ntok, Prof *prof,
+bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b0, int rows, int ntok, Prof *prof,
                         const SolveBuffers *pool = nullptr) {
     const Dims &D = c->D;
     const int d = D.d, H = D.H;
@@ -378,6 +378,12 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
     // W_o on the fp16-split ring tiles reads its A (mix) pre-split: the attention writes the
     // halves, in mix's memory, with the scale the GEMM derives from the h bound (set_range below)
     const bool wo_pre = gemm_wo_presplit(c->prec, rows, d, H);
+    // No token can exit before the last iteration: list 0 serves them all, and neither its count
+    // nor (for a whole forward's list 0, 1, 2, ...) its entries are read on the device
+    const bool all = !(r.eps > 0.0f) && !b0.rprev && m == 0;
+    SolveBuffers b = b0;
+    b.all_rows = all ? rows : 0;
+    b.ident = all && rows == ntok;
     SolveBuffers ba = b;
     if (wo_pre) {
         ba.mix_pre = b.mix;
@@ -390,13 +396,12 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
     // at the last iteration, where it records the iteration counts.  The iterates alternate
     // between two small buffers (a product's column blocks read h_{k-1} while the slot's first
     // block writes h_k), and the active list stays list 0.
-    const bool fixed = gemm_attn_fusable(c->prec, rows, d, H) && rows == ntok && !(r.eps > 0.0f) &&
-                       !b.rprev && m == 0 && !b.mem_hist && r.max_iters >= 2;
+    const bool fixed = gemm_attn_fusable(c->prec, rows, d, H) && rows == ntok && all && !b.mem_hist && r.max_iters >= 2;
     const long fix_stride = (long)std::min<long>(c->cap_tok, ATTN_FUSE_ROWS) * H * d;
     const bool pool_here = fixed && pool && (long)H * d <= 16384;  // the update's LDS holds a token's rows
     auto iterate = [&](int j) { return j == 0 ? b.h : c->fix_h + (long)(j & 1) * fix_stride; };
     for (int k = 0; k < r.max_iters; ++k) {
-        const int cur = fixed ? 0 : k & 1;
+        const int cur = all ? 0 : k & 1;
         {  // Q|K|V for every slot of every active token
             GemmParams g{};
             g.role = ROLE_QKV;
@@ -410,7 +415,7 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
                 g.upd_beta = r.damping;
                 g.upd_excl = (D.flags & ADN_F_RMS_EXCL_ANCHOR) != 0;
             }
-            g.a_idx = b.act[cur];
+            g.a_idx = b.ident ? nullptr : b.act[cur];
             g.a_idx_max = ntok;
             g.a_sm = (long)H * d;
             g.a_ss = d;
@@ -426,7 +431,7 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
             g.N = 3 * d;
             g.K = d;
             g.S = H;
-            g.m_count = b.cnt + cur;
+            g.m_count = all ? nullptr : b.cnt + cur;
             g.err = b.err;
             g.epi = c->qk_bias ? EPI_BIAS : EPI_NONE;
             set_split(c, g, c->sp_qkv);
@@ -456,7 +461,7 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
             g.N = d;
             g.K = d;
             g.S = H;
-            g.m_count = b.cnt + cur;
+            g.m_count = all ? nullptr : b.cnt + cur;
             g.err = b.err;
             g.epi = EPI_NONE;
             set_split(c, g, c->sp_o);
@@ -465,7 +470,7 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b, int
             if (attn_in_wo) {
                 g.attn_qkv = b.qkv;
                 g.attn_clamp = (D.flags & ADN_F_SCORE_CLAMP4) != 0;
-                g.attn_cnt_next = b.cnt + (cur ^ 1);
+                g.attn_cnt_next = all ? nullptr : b.cnt + (cur ^ 1);
                 g.attn_cnt_hist = b.cnt_hist + k;
             }
             Span sp(prof, ADN_STAGE_WO_GEMM, k, st, -1, attn_in_wo ? PROF_FUSED_ATTN : 0);
