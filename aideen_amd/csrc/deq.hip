@@ -21,6 +21,9 @@ constexpr int WAVES_PER_BLOCK = 4;
 // init: h0 = x + anchor (FPMR:1432-1448) or signal/rms(signal) (UWGSL:900-943); first active
 // list = all tokens in order; iteration counts cleared.
 // ---------------------------------------------------------------------------------------
+// VEC consecutive floats per lane: 4 where the caller's rows allow it (32768 tokens of 8 x 512:
+// 223 -> 158 us; the store of h0 is what is left).
+template <int VEC>
 __global__ void k_init(Dims D, SolveBuffers b, const float *x_src, const int32_t *tokens, int ntok,
                        const float *anchor) {
     const int wave = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
@@ -53,7 +56,13 @@ __global__ void k_init(Dims D, SolveBuffers b, const float *x_src, const int32_t
         }
         const float *x = x_src + xr * d;
         const float *an = anchor + (long)s * d;
-        for (int i = lane; i < d; i += 64) put(i, x[i] + an[i]);
+        typedef float vec __attribute__((ext_vector_type(VEC)));
+        for (int i = lane * VEC; i < d; i += 64 * VEC) {
+            const vec v = *reinterpret_cast<const vec *>(x + i) + *reinterpret_cast<const vec *>(an + i);
+            *reinterpret_cast<vec *>(h + i) = v;
+#pragma unroll
+            for (int u = 0; u < VEC; ++u) mx = fmaxf(mx, fabsf(v[u]) < INFINITY ? fabsf(v[u]) : 0.0f);
+        }
     }
     if (b.amax_h) track_absmax(b.amax_h, mx);  // the bound on |h| the split GEMMs scale their A by
     if (s == 0 && lane == 0) {
@@ -150,7 +159,9 @@ __device__ __forceinline__ void store_presplit_pair(float *row, int e0, const fl
 // D.H - 1 again, take no part in the softmax and store nothing.  The padded form replaced a kernel
 // that walked the slots at run time, one wave per query slot with a branch around each load: 6
 // slots of 320 at 4000 tokens 106 -> 40 us, 12 slots of 512 at 900 tokens 66 -> 54.
-template <int H, int QA, int VEC, bool PAD>
+// NC > 0 (one wave per query slot, d = 64 VEC NC): the V rows are loaded beside Q and K, one round
+// trip instead of two where latency is all there is (24 tokens of 8 x 512: 5.8 -> 4.5 us).
+template <int H, int QA, int VEC, bool PAD, int NC>
 __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, int k) {
     static_assert(QA * H <= 64, "the score butterfly leaves one score per lane: at most 64 per wave");
     constexpr int NG = H / QA;
@@ -179,7 +190,36 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
 #pragma unroll
         for (int c = 0; c < H; ++c) part[a][c] = 0.0f;
 
-    for (int off = lane * VEC; off < d; off += 64 * VEC) {
+    float vp[NC ? NC : 1][NC ? H : 1][VEC];
+    if constexpr (NC > 0) {
+        static_assert(QA == 1, "V beside K: one query slot per wave");
+        float q[NC][VEC], kk[NC][H][VEC];
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) q[j][v] = base[(long)slot(g) * rowstride + lane * VEC + 64 * VEC * j + v];
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int c = 0; c < H; ++c)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v)
+                    kk[j][c][v] = base[(long)slot(c) * rowstride + d + lane * VEC + 64 * VEC * j + v];
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int c = 0; c < H; ++c)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v)
+                    vp[j][c][v] = base[(long)slot(c) * rowstride + 2 * d + lane * VEC + 64 * VEC * j + v];
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int c = 0; c < H; ++c)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) part[0][c] += q[j][v] * kk[j][c][v];
+    }
+    for (int off = lane * VEC; NC == 0 && off < d; off += 64 * VEC) {
         float q[QA][VEC];
 #pragma unroll
         for (int a = 0; a < QA; ++a)
@@ -273,7 +313,7 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
 
     float *mixbase = b.mix + (long)i * HR * d;
     const float asc = b.mix_pre ? presplit_scale(b) : 1.0f;
-    for (int off = lane * VEC; off < d; off += 64 * VEC) {
+    auto mix_chunk = [&](int off, int j) {
         float acc[QA][VEC];
 #pragma unroll
         for (int a = 0; a < QA; ++a)
@@ -283,7 +323,8 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
         for (int c = 0; c < H; ++c) {
             float vv[VEC];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) vv[v] = qkv_load<NT>(base + (long)slot(c) * rowstride + 2 * d + off + v);
+            for (int v = 0; v < VEC; ++v)
+                vv[v] = NC ? vp[NC ? j : 0][NC ? c : 0][v] : qkv_load<NT>(base + (long)slot(c) * rowstride + 2 * d + off + v);
 #pragma unroll
             for (int a = 0; a < QA; ++a)
 #pragma unroll
@@ -307,6 +348,12 @@ __global__ __launch_bounds__(256) void k_attn(Dims D, SolveBuffers b, int cur, i
                 for (int v = 0; v < VEC; ++v) mixbase[(long)(g * QA + a) * d + off + v] = acc[a][v];
             }
         }
+    };
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) mix_chunk(lane * VEC + 64 * VEC * j, j);
+    } else {
+        for (int off = lane * VEC; off < d; off += 64 * VEC) mix_chunk(off, 0);
     }
 }
 
@@ -1252,12 +1299,32 @@ void attn_dispatch_vec(const Dims &D, const SolveBuffers &b, int cur, int k, int
     constexpr int NG = H / QA;
     const long waves = (long)ntok * NG;
     const dim3 grid((unsigned)((waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK));
-    if (D.d % 256 == 0)
-        hipLaunchKernelGGL((k_attn<H, QA, 4, PAD>), grid, dim3(256), 0, st, D, b, cur, k);
-    else if (D.d % 128 == 0)
-        hipLaunchKernelGGL((k_attn<H, QA, 2, PAD>), grid, dim3(256), 0, st, D, b, cur, k);
+    auto go = [&](auto Vc, auto Nc) {
+        constexpr int VEC = decltype(Vc)::value, NC = QA == 1 && H * VEC * decltype(Nc)::value <= 64 ? decltype(Nc)::value : 0;
+        hipLaunchKernelGGL((k_attn<H, QA, VEC, PAD, NC>), grid, dim3(256), 0, st, D, b, cur, k);
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using I4 = std::integral_constant<int, 4>;
+    using I0 = std::integral_constant<int, 0>;
+    const int d = D.d;
+    if (d == 256)
+        go(I4(), I1());
+    else if (d == 512)
+        go(I4(), I2());
+    else if (d % 256 == 0)
+        go(I4(), I0());
+    else if (d == 128)
+        go(I2(), I1());
+    else if (d % 128 == 0)
+        go(I2(), I0());
+    else if (d == 64)
+        go(I1(), I1());
+    else if (d == 192)
+        go(I1(), I3());
     else
-        hipLaunchKernelGGL((k_attn<H, QA, 1, PAD>), grid, dim3(256), 0, st, D, b, cur, k);
+        go(I1(), I0());
 }
 
 // One wave per (token, query slot) for few tokens: the same scores, more waves; else QA query slots
@@ -1276,8 +1343,12 @@ void attn_dispatch(const Dims &D, const SolveBuffers &b, int cur, int k, int nto
 void launch_init(const Dims &D, const SolveBuffers &b, const float *x_src, const int32_t *tokens,
                  int ntok, const float *anchor, hipStream_t st) {
     const long waves = (long)ntok * D.H;
-    hipLaunchKernelGGL(k_init, dim3((unsigned)((waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)),
-                       dim3(64 * WAVES_PER_BLOCK), 0, st, D, b, x_src, tokens, ntok, anchor);
+    const dim3 grid((unsigned)((waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)), blk(64 * WAVES_PER_BLOCK);
+    // rows are multiples of 256 bytes; the caller's s_in and h_star may start anywhere
+    if ((((uintptr_t)x_src | (uintptr_t)b.h | (uintptr_t)anchor) & 15) == 0)
+        hipLaunchKernelGGL(k_init<4>, grid, blk, 0, st, D, b, x_src, tokens, ntok, anchor);
+    else
+        hipLaunchKernelGGL(k_init<1>, grid, blk, 0, st, D, b, x_src, tokens, ntok, anchor);
 }
 
 void launch_attn(const Dims &D, const SolveBuffers &b, int cur, int k, int ntok, hipStream_t st) {

@@ -368,8 +368,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN >= 8) ? 1 : 2) void k_ge
     }
 }
 
-// Skinny GEMM (the LM head at most 32 rows, the other products at most ATTN_FUSE_ROWS, which may
-// carry a fused stage: a decode step).  There the
+// Skinny GEMM (at most ATTN_FUSE_ROWS rows, W_o and Q|K|V with a fused stage: a decode step).  There the
 // ring kernel's serial k loop (one barrier per 16-K slice) is the whole cost, so here a
 // workgroup of KW waves owns a 32 x (32 WTN) output block and wave w multiplies its own K range
 // [w K/KW, (w+1) K/KW) straight from global memory into registers, 64 K values per step:
@@ -900,7 +899,7 @@ TilePick pick_tiles(int M, int N, int S) {
 // The LM head's blocks hold whole arg-max partials (128 columns): 64x256 up to 64 rows, 128x128
 // above, both of 32x128 waves, or 256x256 (costs as above); a head too narrow to fill the chip takes
 // 64x128 blocks.  V = 50257, K = 512, A pre-split: 64 rows 38.5 us (128x128 blocks of 64x64 waves) ->
-// 23, 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8 us.
+// 23 (24 rows on the few-row kernel 32 -> 23), 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8 us.
 TilePick pick_lm_tiles(int M, int V) {
     const int nv = (V + 127) / 128;
     if ((M + 127) / 128 * nv < 64) return TP_R64X128;
@@ -949,13 +948,8 @@ void launch_cfg(const GemmParams &p, hipStream_t st) {
     while (steps % kw) kw >>= 1;
     if constexpr (ROLE == ROLE_LMHEAD) {
         if (p.M <= LM_SKINNY_ROWS) {
-            // skinny LM head (a decode step): 128-column blocks, the arg-max partials' width; at
-            // a few rows 64-column blocks with partials per 64 columns (twice the workgroups on
-            // the weight stream)
-            if (gemm_lm_partial_cols(p.prec, p.M, p.K) == 64)
-                launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
-            else
-                launch_skinny<ROLE, T, TERMS, 4>(p, kw, st);
+            // skinny LM head (a decode step): 64-column blocks with arg-max partials per 64 columns
+            launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
             return;
         }
         launch_ring<ROLE, T, TERMS, F16>(p, pick_lm_tiles(p.M, p.N), st);  // fp16: gemm_lm_presplit

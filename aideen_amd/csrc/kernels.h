@@ -103,7 +103,7 @@ struct GemmParams {
     int upd_excl;              // ADN_F_RMS_EXCL_ANCHOR
 };
 constexpr int ATTN_FUSE_ROWS = 4;
-constexpr int LM_SKINNY_ROWS = 32;  // the LM head's few-row kernel
+constexpr int LM_SKINNY_ROWS = ATTN_FUSE_ROWS;  // the LM head's few-row kernel
 constexpr int GEMM_BN = 128;
 void launch_gemm(const GemmParams &p, hipStream_t st);
 void launch_gemm_split(const GemmParams &p, hipStream_t st);
@@ -338,6 +338,9 @@ void launch_fill_i32(int32_t *p, int32_t v, long n, hipStream_t st);
 // the forward may be captured in a graph).
 constexpr int ADN_BOUNDS = 4;
 void launch_reset_bounds(unsigned *words, float h_bound, unsigned *zero, hipStream_t st);  // zero: also cleared, or null
+// launch_reset_bounds and the largest finite |x[i]|, i < n, into *absmax in one block, for few values
+constexpr long BEGIN_SMALL_N = 32768;
+void launch_begin_small(unsigned *words, float h_bound, const float *x, int n, unsigned *absmax, hipStream_t st);
 // ---- memory-coupled solve (memory.hip) -----------------------------------------------------
 // act[0] = tokens (b, t) = b*T + t for b < B, cnt[0] = B, cnt[1] = 0.
 // embed_context of the window ending at every position; tot0/tot1 hold

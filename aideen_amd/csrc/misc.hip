@@ -147,6 +147,33 @@ __global__ void k_reset_bounds(unsigned *words, unsigned w0, unsigned *zero) {
     if (i == ADN_BOUNDS && zero) *zero = 0u;
 }
 
+// The reset and the magnitude of a small call's input in one launch (d = 192, 128 rows: 4.6 + 7.6 us
+// in two, 5 in one); 16 loads in flight per thread.
+__global__ __launch_bounds__(1024) void k_begin_small(unsigned *words, unsigned w0, const float *x, int n,
+                                                      unsigned *absmax) {
+    __shared__ unsigned part[16];
+    unsigned m = 0;
+    for (int i0 = threadIdx.x; i0 < n; i0 += 16 * 1024) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = x[min(i0 + 1024 * u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const float a = fabsf(v[u]);
+            if (a < INFINITY) m = max(m, __float_as_uint(a));
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, 64));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x < ADN_BOUNDS) words[threadIdx.x] = threadIdx.x == 0 ? w0 : 0u;
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) m = max(m, part[w]);
+        *absmax = m;
+    }
+}
+
 // The GPU spectral renormalisation (spectral_renorm.wgsl:83-196): one workgroup of 256 per matrix.
 // The shader indexes its buffer as wg[i*d + j]; with the matrix M as stored here (row-major
 // [d][d]) that buffer is M^T (RENORM_T, the per-slot Q/K/V/O and W_out, whose reference buffers
@@ -228,6 +255,12 @@ void launch_reset_bounds(unsigned *words, float h_bound, unsigned *zero, hipStre
     unsigned bits;
     memcpy(&bits, &h_bound, sizeof bits);
     hipLaunchKernelGGL(k_reset_bounds, dim3(1), dim3(64), 0, st, words, bits, zero);
+}
+
+void launch_begin_small(unsigned *words, float h_bound, const float *x, int n, unsigned *absmax, hipStream_t st) {
+    unsigned bits;
+    memcpy(&bits, &h_bound, sizeof bits);
+    hipLaunchKernelGGL(k_begin_small, dim3(1), dim3(1024), 0, st, words, bits, x, n, absmax);
 }
 
 void launch_spectral_norm(const float *w, int rows, int cols, int n_iter, float *sigma, float *work,

@@ -325,7 +325,13 @@ void enqueue_signal_init(adn_ctx *c, const adn_run &r, const SolveBuffers &b, in
     // caller-supplied rows on the fp16 split: the signal GEMM's A scale also honours their actual
     // magnitude (max |s_in|, accumulated into c->absmax, which the reset clears)
     const bool dyn_scale = r.s_in && c->prec == PREC_F16X3;
-    if (!s_in_ready) launch_reset_bounds(c->bounds, c->h_bound, dyn_scale ? c->absmax : nullptr, st);
+    const bool small = dyn_scale && (long)ntok * d <= BEGIN_SMALL_N;
+    if (!s_in_ready) {
+        if (small)
+            launch_begin_small(c->bounds, c->h_bound, r.s_in, ntok * d, c->absmax, st);
+        else
+            launch_reset_bounds(c->bounds, c->h_bound, dyn_scale ? c->absmax : nullptr, st);
+    }
     // x gathered from the embedding when tokens are given
     {
         GemmParams g{};
@@ -351,7 +357,7 @@ void enqueue_signal_init(adn_ctx *c, const adn_run &r, const SolveBuffers &b, in
         if (dyn_scale) {
             // rows of any size stay inside the fp16 range (rows no larger than the embedding
             // table's entries keep the embedding's scale, and match the token path bit for bit)
-            if (!s_in_ready) launch_absmax(r.s_in, (long)ntok * d, c->absmax, st);
+            if (!s_in_ready && !small) launch_absmax(r.s_in, (long)ntok * d, c->absmax, st);
             g.a_absmax = c->absmax;
             g.a_headroom = 1024.0f;
         }
