@@ -924,9 +924,19 @@ void launch_ring(const GemmParams &p, TilePick tp, hipStream_t st) {
             hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 2, 2, 4, PRE>), dim3(tiles(p, 64, 256)), dim3(256), 0, st, p);
             break;
         case TP_R128:
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
-            break;
-        default: {
+            if (TERMS == 3 || tiles(p, 128, 256) < 192) {
+                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
+                break;
+            }
+            [[fallthrough]];
+        default:
+        if constexpr (TERMS == 1) {
+            // One product per tile leaves little matrix work between a slice's barriers, so two
+            // workgroups per CU (64 KB of ring each) beat one: 128x256 blocks of 64x128 waves, bf16
+            // Q|K|V of 6000 rows 130 us on 256x256 blocks -> 113, W_o 51 -> 45, 2048 LM-head rows
+            // 234 -> 207 (224 on 128x128).  With three products the ring leaves room for one.
+            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 2, 2, 4, PRE>), dim3(tiles(p, 128, 256)), dim3(256), 0, st, p);
+        } else {
             const int grid = ring_grid(tiles(p, 256, 256), 1);
             if constexpr (ROLE == ROLE_QKV)
                 // waves of 32 x 256 (8 down the block): each A row block is split by one wave only

@@ -65,3 +65,24 @@ def test_token_limits_match_oracle(d, H, n):
     ref = pyoracle.Oracle(mc, w).forward(ids[None].astype(np.int32), nthreads=8, want_scan=False)
     np.testing.assert_allclose(got["h_star"][0], ref["h_star"][0][inv], rtol=RTOL, atol=ATOL)
     assert (got["iters"] == 2).all()
+
+
+@pytest.mark.parametrize("shape", [(128, 8, 257, 1, 1500), (256, 16, 1025, 3, 331)], ids=lambda s: "x".join(map(str, s)))
+def test_bf16_blocks_match_fp32_gemms(shape):
+    """bf16-input products on the 128x256 blocks (a partial last row and column block) against the
+    fp32 products of the same model: one bf16 rounding of each operand, 2^-8 relative a product, well
+    inside 2e-2 of outputs of order one after two contracting steps."""
+    d, H, V, B, T = shape
+    toks = synth.make_tokens("uniform", B, T, V, seed=1)
+    got = {}
+    for f in (synth.F_GEMM_BF16, synth.F_GEMM_FP32):
+        mc = synth.ModelConfig(d=d, H=H, V=V, N=1, max_iters=2, eps=0.0, flags=synth.F_SCAN_SELECTIVE | f)
+        be = GpuDeqBackend(mc, B, T)
+        be.upload_weights(synth.make_token_sensitive_weights(mc))
+        got[f] = be.forward(toks, want=("h_star", "logits", "argmax"))
+        be.close()
+    a, b = got[synth.F_GEMM_BF16], got[synth.F_GEMM_FP32]
+    for k in ("h_star", "logits"):
+        assert np.abs(a[k] - b[k]).max() <= 2e-2 * max(1.0, np.abs(b[k]).max()), k
+    lg = a["logits"].reshape(-1, V)
+    assert np.array_equal(a["argmax"].ravel(), V - 1 - np.argmax(lg[:, ::-1], axis=1))
