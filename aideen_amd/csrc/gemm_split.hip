@@ -876,16 +876,19 @@ void launch_skinny(const GemmParams &p, int kw, hipStream_t st) {
 //   256x256 ring, persistent        192 blocks 47.7 us,  768 blocks 157,   1536 blocks 300
 // The 256x256 blocks do the least work per value, and lose where their last round is nearly empty:
 // 1500 rows of Q|K|V (288 blocks) 85 us against 66 on 128x128 blocks, W_o 34 against 22.
+// Products that an exit test follows (GemmParams::exits) take the ring kernel's tiles only, which all
+// sum K in one chain: a 256-row window's iteration counts moved by one step for 3 of 256 tokens where
+// W_o and W_in were K-sliced.
 enum TilePick { TP_KS32, TP_KS32X64, TP_KS64, TP_R64X128, TP_R64X256, TP_R128, TP_R256 };
-TilePick pick_tiles(int M, int N, int S) {
+TilePick pick_tiles(int M, int N, int S, bool exits) {
     static const struct {
         int bm, bn;
         float a, b;
     } cf[] = {{32, 32, 3.0f, 2.6f}, {32, 64, 4.0f, 3.5f}, {64, 64, 5.0f, 6.5f},     {64, 128, 3.0f, 8.7f},
               {64, 256, 5.5f, 13.0f}, {128, 128, 5.0f, 13.0f}, {256, 256, 3.0f, 46.0f}};
-    int best = 0;
+    int best = TP_R64X128;
     float least = INFINITY;
-    for (int i = 0; i < 7; ++i) {
+    for (int i = exits ? TP_R64X128 : TP_KS32; i < 7; ++i) {
         const long n = (long)((M + cf[i].bm - 1) / cf[i].bm) * ((N + cf[i].bn - 1) / cf[i].bn) * S;
         const float t = cf[i].a + cf[i].b * (i < TP_R64X128 ? (float)n / 256.0f : (float)((n + 255) / 256));
         if (t < least) {
@@ -990,7 +993,15 @@ void launch_cfg(const GemmParams &p, hipStream_t st) {
             hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 1, 4>), dim3(tiles(p, 128, 64)), dim3(128), 0, st, p);
             return;
         }
-        const TilePick tp = pick_tiles(p.M, p.N, p.S);
+        if (p.exits && p.M <= FEW_ROWS) {
+            // two column tiles per wave for wide outputs (each A fragment feeds both; 32 rows: 7%)
+            if (p.N >= 1024)
+                launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
+            else
+                launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
+            return;
+        }
+        const TilePick tp = pick_tiles(p.M, p.N, p.S, p.exits);
         switch (tp) {
             case TP_KS32: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 8, 1, 1>), dim3(tiles(p, 32, 32)), dim3(512), 0, st, p); return;
             case TP_KS32X64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 1, 2>), dim3(tiles(p, 32, 64)), dim3(256), 0, st, p); return;
@@ -1029,8 +1040,9 @@ void launch_gemm_split(const GemmParams &p, hipStream_t st) {
     }
 }
 
-bool gemm_wo_presplit(int prec, int M, int N, int S) {
-    return prec == PREC_F16X3 && M > ATTN_FUSE_ROWS && !(N <= 64 && M >= 1024) && pick_tiles(M, N, S) >= TP_R64X128;
+bool gemm_wo_presplit(int prec, int M, int N, int S, bool exits) {
+    return prec == PREC_F16X3 && M > (exits ? FEW_ROWS : ATTN_FUSE_ROWS) && !(N <= 64 && M >= 1024) &&
+           pick_tiles(M, N, S, exits) >= TP_R64X128;
 }
 
 bool gemm_lm_presplit(int prec, int M) { return prec == PREC_F16X3 && M > LM_SKINNY_ROWS; }

@@ -80,6 +80,11 @@ struct GemmParams {
     // (k_gemm_split's pre-split layout); W_o and the LM head, for the shapes gemm_wo_presplit and
     // gemm_lm_presplit name; null = none
     const float *a_pre;
+    // An exit test reads what follows from this product (a tolerance or the plateau exit): a token
+    // whose residual lies within rounding of the limit exits one step earlier or later with the
+    // order its sums are taken in.  K is then summed in one order from FEW_ROWS + 1 rows on and in
+    // one from 1 to FEW_ROWS (the ring kernel's and the few-row kernel's), whatever the blocks.
+    int exits;
     // W_o on at most ATTN_FUSE_ROWS rows (the skinny kernel, split arithmetic): with attn_qkv set
     // the A operand (the attention mix of slot s) is formed in the kernel from the compact
     // [row][S][3K] Q|K|V rows instead of read, so no attention kernel runs; the kernel also does
@@ -103,13 +108,14 @@ struct GemmParams {
     int upd_excl;              // ADN_F_RMS_EXCL_ANCHOR
 };
 constexpr int ATTN_FUSE_ROWS = 4;
+constexpr int FEW_ROWS = 32;  // the few-row kernel's block
 constexpr int LM_SKINNY_ROWS = ATTN_FUSE_ROWS;  // the LM head's few-row kernel
 constexpr int GEMM_BN = 128;
 void launch_gemm(const GemmParams &p, hipStream_t st);
 void launch_gemm_split(const GemmParams &p, hipStream_t st);
 // Whether the product reads its A operand pre-split (GemmParams::a_pre): fp16 halves, W_o of M rows
 // and S slots on the ring kernel's tiles, the LM head beyond the skinny kernel's rows.
-bool gemm_wo_presplit(int prec, int M, int N, int S);
+bool gemm_wo_presplit(int prec, int M, int N, int S, bool exits);
 bool gemm_lm_presplit(int prec, int M);
 // Whether W_o on at most M rows runs with the attention formed in its kernel (GemmParams::attn_qkv):
 // the skinny split-arithmetic kernel, M <= ATTN_FUSE_ROWS, K a multiple of 64, at most 16 slots.

@@ -313,6 +313,10 @@ float max_row_l1(const float *w, int H, int d, bool in_out) {
 // ---------------------------------------------------------------------------------------
 // the forward pipeline (device pointers; enqueue only)
 // ---------------------------------------------------------------------------------------
+// Whether a token can exit before the last iteration (Anderson mixing aside, whose lists the
+// iterations keep in any case)
+bool may_exit(const adn_run &r, const SolveBuffers &b) { return r.eps > 0.0f || b.rprev; }
+
 // signal[t][s] = W_in[s] x_t for every token, h0 and the first active list (all tokens).
 // s_in_ready: the bounds were reset and max |s_in| accumulated into c->absmax by the caller's
 // kernels (a decode step: the previous step's arg-max and this step's query); init_done: so was
@@ -352,6 +356,7 @@ void enqueue_signal_init(adn_ctx *c, const adn_run &r, const SolveBuffers &b, in
         g.S = H;
         g.err = b.err;
         g.epi = EPI_NONE;
+        g.exits = may_exit(r, b);
         set_split(c, g, c->sp_in, c->embed_scale);
         Span sp(prof, ADN_STAGE_SIGNAL_GEMM, -1, st);
         if (dyn_scale) {
@@ -381,12 +386,13 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b0, in
     // Anderson depths 1 and 2 never mix (n_res = min(k, m - 1) < 2), so they run as plain Picard
     // (no ring of iterates)
     const int m = c->cfg.anderson_m >= 3 ? c->cfg.anderson_m : 0;
+    const bool exits = may_exit(r, b0);
     // W_o on the fp16-split ring tiles reads its A (mix) pre-split: the attention writes the
     // halves, in mix's memory, with the scale the GEMM derives from the h bound (set_range below)
-    const bool wo_pre = gemm_wo_presplit(c->prec, rows, d, H);
+    const bool wo_pre = gemm_wo_presplit(c->prec, rows, d, H, exits);
     // No token can exit before the last iteration: list 0 serves them all, and neither its count
     // nor (for a whole forward's list 0, 1, 2, ...) its entries are read on the device
-    const bool all = !(r.eps > 0.0f) && !b0.rprev && m == 0;
+    const bool all = !exits && m == 0;
     SolveBuffers b = b0;
     b.all_rows = all ? rows : 0;
     b.ident = all && rows == ntok;
@@ -440,6 +446,7 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b0, in
             g.m_count = all ? nullptr : b.cnt + cur;
             g.err = b.err;
             g.epi = c->qk_bias ? EPI_BIAS : EPI_NONE;
+            g.exits = exits;
             set_split(c, g, c->sp_qkv);
             set_range(c, g, 0);
             Span sp(prof, ADN_STAGE_QKV_GEMM, k, st, -1, g.upd_o ? PROF_FUSED_UPDATE : 0);
@@ -470,6 +477,7 @@ bool enqueue_iterations(adn_ctx *c, const adn_run &r, const SolveBuffers &b0, in
             g.m_count = all ? nullptr : b.cnt + cur;
             g.err = b.err;
             g.epi = EPI_NONE;
+            g.exits = exits;
             set_split(c, g, c->sp_o);
             set_range(c, g, 0, c->l1_wv);  // mix is a convex combination of V = W_v h rows
             if (wo_pre) g.a_pre = b.mix;
@@ -765,6 +773,7 @@ void enqueue_forward_memory(adn_ctx *c, const adn_run &r, const adn_outputs &o, 
             g.S = H;
             g.err = b.err;
             g.epi = EPI_NONE;
+            g.exits = may_exit(r, b);
             set_split(c, g, c->sp_hist);
             set_range(c, g, 2, 1.0f + (c->w_out ? c->l1_wout : 0.0f));  // m_{t-1} = (I + W_out) m_inner
             {
@@ -798,6 +807,7 @@ void enqueue_forward_memory(adn_ctx *c, const adn_run &r, const adn_outputs &o, 
             g.S = H;
             g.err = b.err;
             g.epi = readout_eye(c) ? EPI_NONE : EPI_ADD_A;
+            g.exits = may_exit(r, b);  // the next position's history
             set_split(c, g, c->sp_out);
             set_range(c, g, 2);
             Span sp(prof, ADN_STAGE_READOUT_GEMM, -1, st, B);

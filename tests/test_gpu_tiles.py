@@ -86,3 +86,44 @@ def test_bf16_blocks_match_fp32_gemms(shape):
         assert np.abs(a[k] - b[k]).max() <= 2e-2 * max(1.0, np.abs(b[k]).max()), k
     lg = a["logits"].reshape(-1, V)
     assert np.array_equal(a["argmax"].ravel(), V - 1 - np.argmax(lg[:, ::-1], axis=1))
+
+
+# (d, H, T, few, many): sequences of T tokens solved in batches of `few` and of `many`, both up to 32
+# rows or both above: 256 rows beside 2304 as one document window beside a throughput batch
+EXIT_SHAPES = [(512, 8, 256, 1, 9), (192, 8, 128, 1, 17), (128, 4, 2048, 1, 3), (1024, 16, 177, 1, 3), (320, 6, 9, 5, 40),
+               (256, 8, 5, 1, 6), (64, 16, 1, 5, 32)]
+
+
+@pytest.mark.parametrize("shape", EXIT_SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("flags", [0, synth.F_GEMM_BF16X3, synth.F_GEMM_BF16], ids=["f16x3", "bf16x3", "bf16"])
+def test_exit_steps_do_not_depend_on_the_batch(shape, flags):
+    """Tokens exit on a tolerance: a sequence's fixed points and iteration counts are the same bits
+    whatever else is solved beside it, since a residual within rounding of the tolerance would
+    otherwise move a token by one update."""
+    d, H, T, few, many = shape
+    mc = synth.ModelConfig(d=d, H=H, V=97, N=1, max_iters=16, eps=1e-4, flags=synth.F_SCAN_SELECTIVE | flags)
+    w = synth.make_token_sensitive_weights(mc)
+    toks = synth.make_tokens("uniform", many, T, mc.V, seed=1)
+    be = GpuDeqBackend(mc, many, T)
+    be.upload_weights(w)
+    want = ("h_star", "iters", "converged")
+    a, b = be.forward(toks[:few], want=want), be.forward(toks, want=want)
+    be.close()
+    for k in want:
+        assert np.array_equal(a[k], b[k][:few]), k
+
+
+# batches of `few` and of `many`, their rows (and B * T signal rows) both up to 32 or both above
+@pytest.mark.parametrize("d,H,T,few,many", [(128, 4, 4, 5, 8), (512, 8, 2, 33, 300)])
+def test_memory_exits_do_not_depend_on_the_batch(d, H, T, few, many):
+    """The memory-coupled solve, where a position's history also goes through W_hist and the readout."""
+    mc = synth.ModelConfig(d=d, H=H, V=97, N=1, max_iters=16, eps=1e-4, flags=synth.F_MEMORY)
+    w = {**synth.make_token_sensitive_weights(mc), **synth.make_hist_weights(mc, seed=11, strong=True)}
+    toks = synth.make_tokens("uniform", many, T, mc.V, seed=1)
+    be = GpuDeqBackend(mc, many, T)
+    be.upload_weights(w)
+    want = ("h_star", "iters", "scan_y")
+    a, b = be.forward(toks[:few], want=want), be.forward(toks, want=want)
+    be.close()
+    for k in want:
+        assert np.array_equal(a[k], b[k][:few]), k
