@@ -927,6 +927,13 @@ void launch_ring(const GemmParams &p, TilePick tp, hipStream_t st) {
             hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 2, 2, 4, PRE>), dim3(tiles(p, 64, 256)), dim3(256), 0, st, p);
             break;
         case TP_R128:
+            if constexpr (ROLE == ROLE_READOUT) {
+                // the readout reads rows that the scan has just streamed out: 64x64 waves wait for them
+                // better than 32x128 (whole carrier calls: 531 rows of 16 x 1024 671-676 us on the
+                // latter, 657-660 on these; 600 of 4 x 1024 240 / 235; 512-wide rows alike)
+                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 2, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
+                break;
+            }
             if (TERMS == 3 || tiles(p, 128, 256) < 192) {
                 hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
                 break;
