@@ -899,10 +899,10 @@ TilePick pick_tiles(int M, int N, int S, bool exits) {
     return (TilePick)best;
 }
 
-// The LM head's blocks hold whole arg-max partials (128 columns): 64x256 up to 64 rows, 128x128
+// The LM head's blocks beyond FEW_ROWS hold whole arg-max partials (128 columns): 64x256 up to 64 rows, 128x128
 // above, both of 32x128 waves, or 256x256 (costs as above); a head too narrow to fill the chip takes
 // 64x128 blocks.  V = 50257, K = 512, A pre-split: 64 rows 38.5 us (128x128 blocks of 64x64 waves) ->
-// 23 (24 rows on the few-row kernel 32 -> 23), 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8 us.
+// 23, 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8 us.
 TilePick pick_lm_tiles(int M, int V) {
     const int nv = (V + 127) / 128;
     if ((M + 127) / 128 * nv < 64) return TP_R64X128;
@@ -967,9 +967,16 @@ void launch_cfg(const GemmParams &p, hipStream_t st) {
     int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
     while (steps % kw) kw >>= 1;
     if constexpr (ROLE == ROLE_LMHEAD) {
-        if (p.M <= LM_SKINNY_ROWS) {
-            // skinny LM head (a decode step): 64-column blocks with arg-max partials per 64 columns
-            launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
+        if (p.M <= FEW_ROWS) {
+            // skinny LM head (a decode or serving step): 128-column blocks, the arg-max partials' width;
+            // at a few rows 64-column blocks with partials per 64 columns (twice the workgroups on the
+            // weight stream).  24 rows x 50257 take 32 us, 28 on the ring kernel's 64x256 blocks, whose
+            // single K chain is further from the exact sum than the four shares here (logits of a
+            // 24-query step 3.1e-7 against 2.5e-7).
+            if (gemm_lm_partial_cols(p.prec, p.M, p.K) == 64)
+                launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
+            else
+                launch_skinny<ROLE, T, TERMS, 4>(p, kw, st);
             return;
         }
         launch_ring<ROLE, T, TERMS, F16>(p, pick_lm_tiles(p.M, p.N), st);  // fp16: gemm_lm_presplit
@@ -1052,7 +1059,7 @@ bool gemm_wo_presplit(int prec, int M, int N, int S, bool exits) {
            pick_tiles(M, N, S, exits) >= TP_R64X128;
 }
 
-bool gemm_lm_presplit(int prec, int M) { return prec == PREC_F16X3 && M > LM_SKINNY_ROWS; }
+bool gemm_lm_presplit(int prec, int M) { return prec == PREC_F16X3 && M > FEW_ROWS; }
 
 int gemm_lm_partial_cols(int prec, int M, int K) {
     return (prec != PREC_FP32 && M <= ATTN_FUSE_ROWS && K % 64 == 0) ? 64 : GEMM_BN;

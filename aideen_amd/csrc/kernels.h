@@ -108,13 +108,12 @@ struct GemmParams {
     int upd_excl;              // ADN_F_RMS_EXCL_ANCHOR
 };
 constexpr int ATTN_FUSE_ROWS = 4;
-constexpr int FEW_ROWS = 32;  // the few-row kernel's block
-constexpr int LM_SKINNY_ROWS = ATTN_FUSE_ROWS;  // the LM head's few-row kernel
+constexpr int FEW_ROWS = 32;  // the few-row kernel's block: the LM head, and products that an exit test follows
 constexpr int GEMM_BN = 128;
 void launch_gemm(const GemmParams &p, hipStream_t st);
 void launch_gemm_split(const GemmParams &p, hipStream_t st);
 // Whether the product reads its A operand pre-split (GemmParams::a_pre): fp16 halves, W_o of M rows
-// and S slots on the ring kernel's tiles, the LM head beyond the skinny kernel's rows.
+// and S slots on the ring kernel's tiles, the LM head beyond FEW_ROWS.
 bool gemm_wo_presplit(int prec, int M, int N, int S, bool exits);
 bool gemm_lm_presplit(int prec, int M);
 // Whether W_o on at most M rows runs with the attention formed in its kernel (GemmParams::attn_qkv):

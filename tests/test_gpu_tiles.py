@@ -127,3 +127,19 @@ def test_memory_exits_do_not_depend_on_the_batch(d, H, T, few, many):
     be.close()
     for k in want:
         assert np.array_equal(a[k], b[k][:few]), k
+
+
+@pytest.mark.parametrize("d,V", [(192, 300), (512, 8300), (1024, 515)])
+def test_few_row_logits_do_not_depend_on_the_batch(d, V):
+    """The LM head up to 32 rows sums K in one order, the shares of the few-row kernel's waves: a
+    row's logits are the same bits at 3, 24 and 32 rows.  One slot and an exit test, so that
+    everything before the head is the same bits too (the softmax over one slot is 1)."""
+    mc = synth.ModelConfig(d=d, H=1, V=V, N=1, max_iters=3, eps=1e-4)
+    toks = synth.make_tokens("uniform", 32, 1, V, seed=1)
+    be = GpuDeqBackend(mc, 32, 1)
+    be.upload_weights(synth.make_token_sensitive_weights(mc))
+    got = [be.forward(toks[:n], want=("pooled", "logits", "argmax")) for n in (3, 24, 32)]
+    be.close()
+    for g in got[1:]:
+        for k in ("pooled", "logits", "argmax"):
+            assert np.array_equal(g[k][:3], got[0][k]), k
