@@ -49,7 +49,8 @@ def test_tiles_match_oracle(shape, flags):
 # tokens on both sides of the attention's and the update's few-token limits, padded slot counts and
 # rows beyond 1024 floats
 @pytest.mark.parametrize("d,H,n", [(64, 3, 385), (128, 5, 641), (64, 8, 1024), (64, 8, 1025), (192, 12, 128),
-                                   (128, 12, 129), (64, 16, 256), (64, 16, 257), (320, 6, 1030), (1024, 16, 40),
+                                   (128, 12, 129), (64, 16, 256), (64, 16, 257), (320, 6, 1030), (320, 8, 24),
+                                   (384, 5, 70), (448, 8, 33), (448, 16, 9), (512, 6, 24), (1024, 16, 40),
                                    (1536, 3, 70), (2048, 2, 129), (2048, 9, 12)])
 def test_token_limits_match_oracle(d, H, n):
     from oracle import pyoracle
