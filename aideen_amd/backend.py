@@ -57,6 +57,16 @@ def device_count() -> int:
     return n.value
 
 
+def gemm_blocks(model, stage: str, rows: int, exits: bool) -> tuple:
+    """Diagnostics (host-only): (rows, columns, waves its inner dimension is divided over, 1 where its
+    input arrives pre-split) of the blocks that a forward's product of `rows` rows runs on; stage is
+    one of ``_lib.STAGES``' products, exits whether an exit test may end the solve."""
+    cfg = AdnConfig(model.d, model.H, model.V, model.N, model.r, 1, 1, model.anderson_m, model.flags)
+    out = (C.c_int32 * 4)()
+    check(lib().adn_gemm_blocks(C.byref(cfg), _lib.STAGES.index(stage), int(rows), int(exits), out))
+    return tuple(out)
+
+
 class GpuDeqBackend:
     """One context on the current HIP device (single-threaded, like the reference backend)."""
 

@@ -65,10 +65,10 @@ __device__ __forceinline__ void load_rows(float (&x)[CHK][DPT], const float *E, 
     if (bad && threadIdx.x == 0) atomicOr(err, ADN_DEVERR_TOKEN);
 }
 
-template <int DPT, int CHK>
 // busy (or null): the overlap guard of a shared chunk-total array, [0] the calls in flight, [1] the
 // window kernel's finished blocks.  The chunk kernel raises [0] (a call that finds it raised
 // overlaps another: ADN_DEVERR_OVERLAP), the last block of the window kernel lowers it.
+template <int DPT, int CHK>
 __global__ __launch_bounds__(ENT) void k_ctx_chunks(const float *E, int d, int V, const int32_t *tokens, int T,
                                                      int nch, double *tot0, double *tot1, unsigned *err,
                                                      unsigned *busy) {

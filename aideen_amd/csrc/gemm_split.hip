@@ -32,10 +32,11 @@
 // fetches the chunk that belongs at its LDS position.
 //
 // Each wave owns WTM x WTN MFMA tiles of 32x32 (v_mfma_f32_32x32x16), the workgroup a WGM x WGN
-// grid of waves.  Wide GEMMs use 256x256 blocks of 8 waves (64x128 each, 2 waves per SIMD; the
-// Q|K|V product 32x256 each, so that every A row block is split by one wave), run persistent: a
-// resident workgroup per CU walks its share of the tiles, loading the next tile's first slices
-// while the current tile's results are stored.
+// grid of waves (pick_blocks chooses them by the product's sizes).  The largest three-product
+// GEMMs use 256x256 blocks of 8 waves (64x128 each, 2 waves per SIMD; the Q|K|V product 32x256
+// each, so that every A row block is split by one wave), run persistent: a resident workgroup per
+// CU walks its share of the tiles, loading the next tile's first slices while the current tile's
+// results are stored.  The largest single-product GEMMs use 128x256 blocks, a workgroup per tile.
 #include "gemm_common.h"
 
 namespace adn {
@@ -368,8 +369,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN >= 8) ? 1 : 2) void k_ge
     }
 }
 
-// Skinny GEMM (at most ATTN_FUSE_ROWS rows, W_o and Q|K|V with a fused stage: a decode step).  There the
-// ring kernel's serial k loop (one barrier per 16-K slice) is the whole cost, so here a
+// Skinny GEMM: every product of at most ATTN_FUSE_ROWS rows (W_o and Q|K|V there with a fused
+// stage: a decode step), the LM head and the products that an exit test follows up to FEW_ROWS.
+// There the ring kernel's serial k loop (one barrier per 16-K slice) is the whole cost, so here a
 // workgroup of KW waves owns a 32 x (32 WTN) output block and wave w multiplies its own K range
 // [w K/KW, (w+1) K/KW) straight from global memory into registers, 64 K values per step:
 // lane (q = lane & 31, g = lane >> 5) loads the 32 consecutive K values [64i + 32g, +32) of A
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN >= 8) ? 1 : 2) void k_ge
 // and summation order: one wave per row, a lane's elements lane + 64e summed in e order, then the
 // wave sum) into LDS, so that the update needs no kernel of its own; the slot's first column
 // block also stores the row.  Used only where no token can exit before the last iteration, so
-// that the update's residual and exit test are not needed.
+// that the update's residual and exit test are not needed and row r is token r (a_idx is null).
 template <int ROLE, typename T, int TERMS, int KW, int WTN, bool ATTN = false, bool UPD = false>
 __global__ __launch_bounds__(64 * KW) void k_gemm_skinny(GemmParams p) {
     typedef typename Vec8<T>::type V8;
@@ -517,12 +519,10 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_skinny(GemmParams p) {
         const long hd = (long)p.S * dd;
         const float beta = p.upd_beta, omb = 1.0f - beta;
         for (int r = wave; r < M; r += KW) {  // M <= ATTN_FUSE_ROWS
-            long t = p.a_idx ? (long)p.a_idx[r] : (long)r;
-            if (p.a_idx && (t < 0 || t >= p.a_idx_max)) t = 0;  // flagged below
-            const float *o = p.upd_o + ((long)r * p.S + s) * dd;
-            const float *sg = p.upd_sig + t * hd + (long)s * dd;
+            const float *o = p.upd_o + r * hd + (long)s * dd;
+            const float *sg = p.upd_sig + r * hd + (long)s * dd;
             const float *an = p.upd_anchor + (long)s * dd;
-            const float *hp = p.A + t * hd + (long)s * dd;
+            const float *hp = p.A + r * hd + (long)s * dd;
             float ss = 0.0f;
             for (int e0 = 0; e0 < E; e0 += 8) {  // 8 elements' loads in flight per lane
                 float ov[8], sv[8], av[8], hv[8], gv[8];
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_skinny(GemmParams p) {
             }
             ss = wave_sum(ss);
             const float rms = sqrtf(ss / (float)dd + 1e-6f);
-            float *hw = p.upd_hout + t * hd + (long)s * dd;
+            float *hw = p.upd_hout + r * hd + (long)s * dd;
             for (int e = 0; e < E; ++e) {  // each lane reads back only what it wrote
                 const int idx = lane + 64 * e;
                 const float f = mix_l[r][idx] / rms;
@@ -664,8 +664,9 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_skinny(GemmParams p) {
 // partial blocks are exchanged through LDS once, each wave then summing (in wave order) and storing
 // 1/KW of the block.  Lane (q = lane & 31, g = lane >> 5) loads K values [8g, 8g + 8) of a step of
 // A row q and B row q: one contiguous kilobyte of B per load, half lines of A.
-// Measured in back-to-back launches, K = 512, 8 slots, against the tiles used before: W_o at 64 rows 17.5 -> 5.3 us, at 256 rows 17.8 -> 10.2; Q|K|V at 64 rows 18.8 -> 9.6;
-// at 24 rows W_o 5.2 -> 4.9 and Q|K|V 6.7 -> 6.0 (the few-row kernel above).
+// Measured in back-to-back launches, K = 512, 8 slots, against the tiles used before: W_o at 64
+// rows 17.5 -> 5.3 us, at 256 rows 17.8 -> 10.2; Q|K|V at 64 rows 18.8 -> 9.6; at 24 rows W_o
+// 5.2 -> 4.9 and Q|K|V 6.7 -> 6.0 (the few-row kernel above).
 template <typename T, int TERMS, int KW, int WTM, int WTN>
 __global__ __launch_bounds__(64 * KW, KW == 8 ? 4 : (WTM == 2 ? 2 : 4)) void k_gemm_ks(GemmParams p) {
     typedef typename Vec8<T>::type V8;
@@ -864,9 +865,26 @@ void launch_skinny(const GemmParams &p, int kw, hipStream_t st) {
     }
 }
 
-// Tiles of a product of M rows: the configuration with the least a + b * (its blocks / 256), for the
-// ring kernels rounded up to whole rounds of one block per CU (the K-sliced blocks are small enough
-// to fill in); us for K = 512 (other K scale all of them alike), fitted to back-to-back launches of 8- and 16-slot products at 5 to 8192 rows, N = 64 to 3072:
+// Blocks of a product.  From R64X128 on the ring kernel, whose blocks all sum K in one chain.
+enum TilePick {
+    TP_FEW,     // k_gemm_skinny: 32 rows, K over its waves
+    TP_NARROW,  // ring, 128x64, two 64x64 waves
+    TP_KS32,    // k_gemm_ks: 32x32, K over 8 waves
+    TP_KS32X64,  // 32x64, K over 4 waves
+    TP_KS64,    // 64x64, K over 4 waves
+    TP_R64X128,   // four 32x64 waves
+    TP_R64X256,   // four 32x128 waves
+    TP_R128,      // 128x128, four 32x128 waves (the readout: 64x64)
+    TP_R128X256,  // four 64x128 waves (single products)
+    TP_R256       // 256x256, eight waves, persistent (three products)
+};
+
+long blocks(int M, int N, int S, int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * S; }
+
+// The configuration with the least a + b * (its blocks / 256), for the ring kernels rounded up to
+// whole rounds of one block per CU (the K-sliced blocks are small enough to fill in); us for
+// three products and K = 512, fitted to back-to-back launches of 8- and 16-slot products at 5 to
+// 8192 rows, N = 64 to 3072:
 //   32x32   K-sliced over 8 waves   256 blocks  5.2 us,  768 blocks  10.0, 1536 blocks  18.6
 //   32x64   K-sliced over 4 waves   256 blocks  7.0 us,  768 blocks  14.1, 1536 blocks  24.4
 //   64x64   K-sliced over 4 waves   256 blocks 10.4 us,  768 blocks  23.6, 1024 blocks  30.1
@@ -876,84 +894,105 @@ void launch_skinny(const GemmParams &p, int kw, hipStream_t st) {
 //   256x256 ring, persistent        192 blocks 47.7 us,  768 blocks 157,   1536 blocks 300
 // The 256x256 blocks do the least work per value, and lose where their last round is nearly empty:
 // 1500 rows of Q|K|V (288 blocks) 85 us against 66 on 128x128 blocks, W_o 34 against 22.
-// Products that an exit test follows (GemmParams::exits) take the ring kernel's tiles only, which all
-// sum K in one chain: a 256-row window's iteration counts moved by one step for 3 of 256 tokens where
-// W_o and W_in were K-sliced.
-enum TilePick { TP_KS32, TP_KS32X64, TP_KS64, TP_R64X128, TP_R64X256, TP_R128, TP_R256 };
+// The order of the costs is K = 512's.  At K = 256 the choice stays within 15% of the best; at K =
+// 2048, where the ring blocks walk four times the slices and the K-sliced ones share them, it is up to
+// 28% off (300 rows x 2 slots: 64x128 53 us, 32x64 42).  Single products change sides at the same row
+// counts (W_o, 8 slots of 512: 200 rows K-sliced 8.7 us, ring 10.2; 300 rows 11.1 / 10.4).
+// Products that an exit test follows (GemmParams::exits) take the ring's tiles only: a 256-row
+// window's iteration counts moved by one step for 3 of 256 tokens where W_o and W_in were K-sliced.
 TilePick pick_tiles(int M, int N, int S, bool exits) {
     static const struct {
+        TilePick tp;
         int bm, bn;
         float a, b;
-    } cf[] = {{32, 32, 3.0f, 2.6f}, {32, 64, 4.0f, 3.5f}, {64, 64, 5.0f, 6.5f},     {64, 128, 3.0f, 8.7f},
-              {64, 256, 5.5f, 13.0f}, {128, 128, 5.0f, 13.0f}, {256, 256, 3.0f, 46.0f}};
-    int best = TP_R64X128;
+    } cf[] = {{TP_KS32, 32, 32, 3.0f, 2.6f},      {TP_KS32X64, 32, 64, 4.0f, 3.5f},  {TP_KS64, 64, 64, 5.0f, 6.5f},
+              {TP_R64X128, 64, 128, 3.0f, 8.7f},  {TP_R64X256, 64, 256, 5.5f, 13.0f}, {TP_R128, 128, 128, 5.0f, 13.0f},
+              {TP_R256, 256, 256, 3.0f, 46.0f}};
+    TilePick best = TP_R64X128;
     float least = INFINITY;
-    for (int i = exits ? TP_R64X128 : TP_KS32; i < 7; ++i) {
-        const long n = (long)((M + cf[i].bm - 1) / cf[i].bm) * ((N + cf[i].bn - 1) / cf[i].bn) * S;
-        const float t = cf[i].a + cf[i].b * (i < TP_R64X128 ? (float)n / 256.0f : (float)((n + 255) / 256));
+    for (const auto &c : cf) {
+        if (exits && c.tp < TP_R64X128) continue;
+        const long n = blocks(M, N, S, c.bm, c.bn);
+        const float t = c.a + c.b * (c.tp < TP_R64X128 ? (float)n / 256.0f : (float)((n + 255) / 256));
         if (t < least) {
             least = t;
-            best = i;
+            best = c.tp;
         }
     }
-    return (TilePick)best;
+    return best;
 }
 
-// The LM head's blocks beyond FEW_ROWS hold whole arg-max partials (128 columns): 64x256 up to 64 rows, 128x128
-// above, both of 32x128 waves, or 256x256 (costs as above); a head too narrow to fill the chip takes
-// 64x128 blocks.  V = 50257, K = 512, A pre-split: 64 rows 38.5 us (128x128 blocks of 64x64 waves) ->
-// 23, 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8 us.
+// The LM head's blocks beyond FEW_ROWS hold whole arg-max partials (128 columns): 64x256 up to 64
+// rows, 128x128 above, both of 32x128 waves, or 256x256 (costs as above); a head too narrow to fill
+// the chip takes 64x128 blocks.  V = 50257, K = 512, A pre-split: 64 rows 38.5 us (128x128 blocks of
+// 64x64 waves) -> 23, 531 rows 168 -> 107, 1024 rows 209 (256x256) -> 176; V = 65, K = 192: 15.8 -> 9.8.
 TilePick pick_lm_tiles(int M, int V) {
-    const int nv = (V + 127) / 128;
-    if ((M + 127) / 128 * nv < 64) return TP_R64X128;
+    if (blocks(M, V, 1, 128, 128) < 64) return TP_R64X128;
     if (M <= 64) return TP_R64X256;
-    const int r128 = ((M + 127) / 128 * nv + 255) / 256, r256 = ((M + 255) / 256 * ((V + 255) / 256) + 255) / 256;
-    return 5.0f + 13.0f * r128 < 3.0f + 46.0f * r256 ? TP_R128 : TP_R256;
+    const long r128 = (blocks(M, V, 1, 128, 128) + 255) / 256, r256 = (blocks(M, V, 1, 256, 256) + 255) / 256;
+    return 5.0f + 13.0f * (float)r128 < 3.0f + 46.0f * (float)r256 ? TP_R128 : TP_R256;
 }
 
-int tiles(const GemmParams &p, int bm, int bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.S; }
+TilePick pick_blocks(int role, int prec, int M, int N, int S, bool exits) {
+    if (M <= ATTN_FUSE_ROWS || (M <= FEW_ROWS && (exits || role == ROLE_LMHEAD))) return TP_FEW;
+    // narrow outputs (the carrier's projections, r + 2N = 64 columns): no zero-padded half tile
+    if (role != ROLE_LMHEAD && N <= 64 && M >= 1024) return TP_NARROW;
+    const TilePick tp = role == ROLE_LMHEAD ? pick_lm_tiles(M, N) : pick_tiles(M, N, S, exits);
+    // One product per tile leaves little matrix work between a slice's barriers, so two workgroups
+    // per CU (64 KB of ring each) beat one: 128x256 blocks of 64x128 waves, Q|K|V of 6000 rows 130 us
+    // on 256x256 blocks -> 113, W_o 51 -> 45, 2048 LM-head rows 234 -> 207 (224 on 128x128).  Against
+    // 128x128 blocks (W_o, 8 slots of 512): 144 blocks of 128x256 15.4 / 15.4 us, 192 15.8 / 16.0, 288
+    // 24.6 / 22.1, 384 27.5 / 24.2; at K = 192 the line lies too low (Q|K|V of 3000 rows, 8 slots: 24 us,
+    // 19 on 128x128 blocks).  With three products the ring leaves room for one.
+    if (prec == PREC_BF16X1 && (tp == TP_R256 || (tp == TP_R128 && blocks(M, N, S, 128, 256) >= 192)))
+        return TP_R128X256;
+    return tp;
+}
+
+// K split over the waves of the few-row kernel, about two 64-K steps per wave (every K is a multiple
+// of 64), each wave's K range whole 64-K steps
+int few_waves(int K) {
+    const int steps = K / 64;
+    int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
+    while (steps % kw) kw >>= 1;
+    return kw;
+}
+
+int tiles(const GemmParams &p, int bm, int bn) { return (int)blocks(p.M, p.N, p.S, bm, bn); }
 
 // The ring kernel on the picked blocks (template order WTM, WTN, WGM, WGN, STAGES); PRE: A pre-split
 // by its producer.  The 256x256 blocks run persistent (8 waves, one resident workgroup per CU
-// walking its share of tiles, the next tile's first slices loaded during the epilogue), the smaller
-// ones a workgroup per tile, whose short k loops would otherwise wait on the previous tile's stores.
+// walking its share of tiles, the next tile's first slices loaded during the epilogue), the others
+// a workgroup per tile, whose short k loops would otherwise wait on the previous tile's stores.
 template <int ROLE, typename T, int TERMS, bool PRE>
 void launch_ring(const GemmParams &p, TilePick tp, hipStream_t st) {
+    auto go = [&](auto kernel, int grid, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, st, p);
+    };
     switch (tp) {
-        case TP_R64X128:
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 2, 2, 2, 4, PRE>), dim3(tiles(p, 64, 128)), dim3(256), 0, st, p);
-            break;
-        case TP_R64X256:
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 2, 2, 4, PRE>), dim3(tiles(p, 64, 256)), dim3(256), 0, st, p);
-            break;
+        case TP_R64X128: go(k_gemm_split<ROLE, T, TERMS, 1, 2, 2, 2, 4, PRE>, tiles(p, 64, 128), 256); break;
+        case TP_R64X256: go(k_gemm_split<ROLE, T, TERMS, 1, 4, 2, 2, 4, PRE>, tiles(p, 64, 256), 256); break;
         case TP_R128:
-            if constexpr (ROLE == ROLE_READOUT) {
+            if constexpr (ROLE == ROLE_READOUT)
                 // the readout reads rows that the scan has just streamed out: 64x64 waves wait for them
                 // better than 32x128 (whole carrier calls: 531 rows of 16 x 1024 671-676 us on the
                 // latter, 657-660 on these; 600 of 4 x 1024 240 / 235; 512-wide rows alike)
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 2, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
-                break;
-            }
-            if (TERMS == 3 || tiles(p, 128, 256) < 192) {
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4, PRE>), dim3(tiles(p, 128, 128)), dim3(256), 0, st, p);
-                break;
-            }
-            [[fallthrough]];
-        default:
-        if constexpr (TERMS == 1) {
-            // One product per tile leaves little matrix work between a slice's barriers, so two
-            // workgroups per CU (64 KB of ring each) beat one: 128x256 blocks of 64x128 waves, bf16
-            // Q|K|V of 6000 rows 130 us on 256x256 blocks -> 113, W_o 51 -> 45, 2048 LM-head rows
-            // 234 -> 207 (224 on 128x128).  With three products the ring leaves room for one.
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 2, 2, 4, PRE>), dim3(tiles(p, 128, 256)), dim3(256), 0, st, p);
-        } else {
-            const int grid = ring_grid(tiles(p, 256, 256), 1);
-            if constexpr (ROLE == ROLE_QKV)
-                // waves of 32 x 256 (8 down the block): each A row block is split by one wave only
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 1, 8, 8, 1, 4, PRE>), dim3(grid), dim3(512), 0, st, p);
+                go(k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 2, 4, PRE>, tiles(p, 128, 128), 256);
             else
-                hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4, PRE>), dim3(grid), dim3(512), 0, st, p);
-        }
+                go(k_gemm_split<ROLE, T, TERMS, 1, 4, 4, 1, 4, PRE>, tiles(p, 128, 128), 256);
+            break;
+        case TP_R128X256:
+            if constexpr (TERMS == 1) go(k_gemm_split<ROLE, T, TERMS, 2, 4, 2, 2, 4, PRE>, tiles(p, 128, 256), 256);
+            break;
+        default:
+            if constexpr (TERMS == 3) {
+                const int grid = ring_grid(tiles(p, 256, 256), 1);
+                if constexpr (ROLE == ROLE_QKV)
+                    // waves of 32 x 256 (8 down the block): each A row block is split by one wave only
+                    go(k_gemm_split<ROLE, T, TERMS, 1, 8, 8, 1, 4, PRE>, grid, 512);
+                else
+                    go(k_gemm_split<ROLE, T, TERMS, 2, 4, 4, 2, 4, PRE>, grid, 512);
+            }
     }
 }
 
@@ -961,65 +1000,54 @@ template <int ROLE, typename T, int TERMS>
 void launch_cfg(const GemmParams &p, hipStream_t st) {
     if (p.M <= 0 || p.N <= 0 || p.S <= 0) return;
     constexpr bool F16 = std::is_same<T, _Float16>::value;
-    // K split over the waves of the few-row kernel, about two 64-K steps per wave (every K is a
-    // multiple of 64), each wave's K range whole 64-K steps
-    const int steps = p.K / 64;
-    int kw = steps >= 16 ? 8 : steps >= 8 ? 4 : steps >= 4 ? 2 : 1;
-    while (steps % kw) kw >>= 1;
-    if constexpr (ROLE == ROLE_LMHEAD) {
-        if (p.M <= FEW_ROWS) {
-            // skinny LM head (a decode or serving step): 128-column blocks, the arg-max partials' width;
-            // at a few rows 64-column blocks with partials per 64 columns (twice the workgroups on the
-            // weight stream).  24 rows x 50257 take 32 us, 28 on the ring kernel's 64x256 blocks, whose
-            // single K chain is further from the exact sum than the four shares here (logits of a
-            // 24-query step 3.1e-7 against 2.5e-7).
+    constexpr bool LM = ROLE == ROLE_LMHEAD;
+    const TilePick tp = pick_blocks(ROLE, p.prec, p.M, p.N, p.S, p.exits);
+    const int kw = few_waves(p.K);
+    if constexpr (LM) {
+        if (tp == TP_FEW) {
+            // a decode or serving step: 128-column blocks, the arg-max partials' width; at a few rows
+            // 64-column blocks with partials per 64 columns (twice the workgroups on the weight
+            // stream).  24 rows x 50257 take 32 us, 28 on the ring kernel's 64x256 blocks, whose single
+            // K chain is further from the exact sum than the four shares here (logits of a 24-query
+            // step 3.1e-7 against 2.5e-7).
             if (gemm_lm_partial_cols(p.prec, p.M, p.K) == 64)
                 launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
             else
                 launch_skinny<ROLE, T, TERMS, 4>(p, kw, st);
             return;
         }
-        launch_ring<ROLE, T, TERMS, F16>(p, pick_lm_tiles(p.M, p.N), st);  // fp16: gemm_lm_presplit
-        return;
+        launch_ring<ROLE, T, TERMS, F16>(p, tp, st);  // fp16: gemm_lm_presplit
     } else {
-        if (p.M <= ATTN_FUSE_ROWS) {
-            // a few rows: one 32-column tile per wave (decode Q|K|V at one row against two tiles:
-            // 248 -> 238 us per token).  The forms with a fused stage and the plain one are the same
-            // product bit for bit.
-            if constexpr (ROLE == ROLE_WO) {
-                if (p.attn_qkv) {  // the attention formed in the kernel
-                    launch_skinny<ROLE, T, TERMS, 1, true>(p, kw, st);
-                    return;
-                }
-            }
-            if constexpr (ROLE == ROLE_QKV) {
-                if (p.upd_o) {  // the previous iteration's update formed in the kernel
-                    launch_skinny<ROLE, T, TERMS, 1, false, true>(p, kw, st);
-                    return;
-                }
-            }
-            launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
-            return;
-        }
-        if (p.N <= 64 && p.M >= 1024) {
-            // narrow outputs (the carrier's projections, r + 2N = 64 columns): 128 x 64 blocks of two
-            // 64 x 64 waves, no zero-padded half tile
-            hipLaunchKernelGGL((k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 1, 4>), dim3(tiles(p, 128, 64)), dim3(128), 0, st, p);
-            return;
-        }
-        if (p.exits && p.M <= FEW_ROWS) {
-            // two column tiles per wave for wide outputs (each A fragment feeds both; 32 rows: 7%)
-            if (p.N >= 1024)
-                launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
-            else
-                launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
-            return;
-        }
-        const TilePick tp = pick_tiles(p.M, p.N, p.S, p.exits);
+        auto go = [&](auto kernel, int grid, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, st, p);
+        };
         switch (tp) {
-            case TP_KS32: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 8, 1, 1>), dim3(tiles(p, 32, 32)), dim3(512), 0, st, p); return;
-            case TP_KS32X64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 1, 2>), dim3(tiles(p, 32, 64)), dim3(256), 0, st, p); return;
-            case TP_KS64: hipLaunchKernelGGL((k_gemm_ks<T, TERMS, 4, 2, 2>), dim3(tiles(p, 64, 64)), dim3(256), 0, st, p); return;
+            case TP_FEW:
+                // The forms with a fused stage and the plain one are the same product bit for bit.  At
+                // a few rows one 32-column tile per wave (decode Q|K|V at one row against two tiles:
+                // 248 -> 238 us per token); above, two for wide outputs (each A fragment feeds both;
+                // 32 rows: 7%).
+                if constexpr (ROLE == ROLE_WO) {
+                    if (p.attn_qkv) {  // the attention formed in the kernel
+                        launch_skinny<ROLE, T, TERMS, 1, true>(p, kw, st);
+                        return;
+                    }
+                }
+                if constexpr (ROLE == ROLE_QKV) {
+                    if (p.upd_o) {  // the previous iteration's update formed in the kernel
+                        launch_skinny<ROLE, T, TERMS, 1, false, true>(p, kw, st);
+                        return;
+                    }
+                }
+                if (p.M > ATTN_FUSE_ROWS && p.N >= 1024)
+                    launch_skinny<ROLE, T, TERMS, 2>(p, kw, st);
+                else
+                    launch_skinny<ROLE, T, TERMS, 1>(p, kw, st);
+                return;
+            case TP_NARROW: go(k_gemm_split<ROLE, T, TERMS, 2, 2, 2, 1, 4>, tiles(p, 128, 64), 128); return;
+            case TP_KS32: go(k_gemm_ks<T, TERMS, 8, 1, 1>, tiles(p, 32, 32), 512); return;
+            case TP_KS32X64: go(k_gemm_ks<T, TERMS, 4, 1, 2>, tiles(p, 32, 64), 256); return;
+            case TP_KS64: go(k_gemm_ks<T, TERMS, 4, 2, 2>, tiles(p, 64, 64), 256); return;
             default: break;
         }
         if constexpr (F16 && ROLE == ROLE_WO) {
@@ -1055,11 +1083,31 @@ void launch_gemm_split(const GemmParams &p, hipStream_t st) {
 }
 
 bool gemm_wo_presplit(int prec, int M, int N, int S, bool exits) {
-    return prec == PREC_F16X3 && M > (exits ? FEW_ROWS : ATTN_FUSE_ROWS) && !(N <= 64 && M >= 1024) &&
-           pick_tiles(M, N, S, exits) >= TP_R64X128;
+    return prec == PREC_F16X3 && pick_blocks(ROLE_WO, prec, M, N, S, exits) >= TP_R64X128;
 }
 
 bool gemm_lm_presplit(int prec, int M) { return prec == PREC_F16X3 && M > FEW_ROWS; }
+
+GemmBlocks gemm_blocks(int role, int prec, int M, int N, int K, int S, bool exits) {
+    if (prec == PREC_FP32) return {GEMM_BN, GEMM_BN, 1, false};
+    const bool lm = role == ROLE_LMHEAD;
+    const TilePick tp = pick_blocks(role, prec, M, N, S, exits);
+    const bool pre = prec == PREC_F16X3 && tp >= TP_R64X128 && (lm || role == ROLE_WO);
+    switch (tp) {
+        case TP_FEW:
+            return {32, lm ? gemm_lm_partial_cols(prec, M, K) : M > ATTN_FUSE_ROWS && N >= 1024 ? 64 : 32, few_waves(K),
+                    false};
+        case TP_NARROW: return {128, 64, 1, false};
+        case TP_KS32: return {32, 32, 8, false};
+        case TP_KS32X64: return {32, 64, 4, false};
+        case TP_KS64: return {64, 64, 4, false};
+        case TP_R64X128: return {64, 128, 1, pre};
+        case TP_R64X256: return {64, 256, 1, pre};
+        case TP_R128: return {128, 128, 1, pre};
+        case TP_R128X256: return {128, 256, 1, pre};
+        default: return {256, 256, 1, pre};
+    }
+}
 
 int gemm_lm_partial_cols(int prec, int M, int K) {
     return (prec != PREC_FP32 && M <= ATTN_FUSE_ROWS && K % 64 == 0) ? 64 : GEMM_BN;

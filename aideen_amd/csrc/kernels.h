@@ -95,10 +95,9 @@ struct GemmParams {
     int32_t *attn_cnt_hist;
     // Q|K|V on at most ATTN_FUSE_ROWS rows (the skinny kernel, split arithmetic) when no token can
     // exit early: with upd_o set the kernel first applies the previous iteration's damped update
-    // to its A rows (A = h before it, K = d, S = H; per slot c = o + signal + anchor, h' =
+    // to its A rows (A = h before it, row r token r, K = d, S = H; per slot c = o + signal + anchor, h' =
     // g c / rms(c) beta + h (1 - beta), as k_update_tok computes it) and multiplies h'; the
-    // slot's first column block writes h' to upd_hout (rows indexed like A).  upd_o is the
-    // previous W_o output, compact by active index like the A index list.
+    // slot's first column block writes h' to upd_hout.  upd_o is the previous W_o output.
     const float *upd_o;
     const float *upd_sig;
     const float *upd_anchor;
@@ -119,6 +118,13 @@ bool gemm_lm_presplit(int prec, int M);
 // Whether W_o on at most M rows runs with the attention formed in its kernel (GemmParams::attn_qkv):
 // the skinny split-arithmetic kernel, M <= ATTN_FUSE_ROWS, K a multiple of 64, at most 16 slots.
 bool gemm_attn_fusable(int prec, int M, int K, int S);
+// Blocks of a product of M rows: rows and columns of one, the waves that its K is divided over (1: one
+// chain), and whether A arrives pre-split (the hist product, a W_o without a_pre, aside).
+struct GemmBlocks {
+    int rows, cols, k_waves;
+    bool pre;
+};
+GemmBlocks gemm_blocks(int role, int prec, int M, int N, int K, int S, bool exits);
 // Columns per arg-max partial of the LM head over M rows (GEMM_BN, or 64 for the few-row skinny
 // LM head): the partial count is ceil(V / this), and the partial buffers hold that many per row.
 int gemm_lm_partial_cols(int prec, int M, int K);
@@ -178,8 +184,9 @@ struct SolveBuffers {
     float *pool_norm;
     const float *pool_g;
     // > 0: no token can exit before the last iteration (a tolerance of zero or less, no plateau
-    // exit), so list 0 with this many rows serves every iteration: its count is not read, nothing
-    // is appended and no residual is formed.  ident: list 0 is 0, 1, 2, ... and is not read either
+    // exit), so list 0 with this many rows serves every iteration: its count is not read and nothing
+    // is appended.  k_update_tok forms no residual then; k_update does and drops it.  ident: list 0
+    // is 0, 1, 2, ... and is not read either
     int all_rows;
     int ident;
     // [ntok][4] the coefficients of each token's last Anderson mix (launch_update_mix), or null

@@ -162,6 +162,13 @@ std::string validate_config(const adn_config &c) {
     return "";
 }
 
+GemmPrec gemm_prec(const adn_config &c) {
+    return (c.flags & ADN_F_GEMM_FP32)     ? PREC_FP32
+           : (c.flags & ADN_F_GEMM_BF16X3) ? PREC_BF16X3
+           : (c.flags & ADN_F_GEMM_BF16)   ? PREC_BF16X1
+                                           : PREC_F16X3;
+}
+
 void upload(adn_ctx *c, float **dst, const float *src, size_t n, const char *name, bool required) {
     if (!src) {
         if (required) throw std::string("missing weight tensor: ") + name;
@@ -883,6 +890,30 @@ int adn_device_count(int32_t *count) {
     return ADN_OK;
 }
 
+int adn_gemm_blocks(const adn_config *cfg, int32_t stage, int32_t rows, int32_t exits, int32_t *blocks) {
+    if (!cfg || !blocks) return fail(ADN_E_INVALID, "null argument");
+    const std::string msg = validate_config(*cfg);
+    if (!msg.empty()) return fail(ADN_E_INVALID, msg);
+    if (rows < 1 || rows > (1 << 24)) return fail(ADN_E_INVALID, "rows must be in [1, 2^24]");
+    const int d = cfg->d_r;
+    int role, N = d, S = cfg->h_slots;
+    switch (stage) {
+        case ADN_STAGE_SIGNAL_GEMM: role = ROLE_SIGNAL; break;
+        case ADN_STAGE_QKV_GEMM: role = ROLE_QKV; N = 3 * d; break;
+        case ADN_STAGE_WO_GEMM:
+        case ADN_STAGE_HIST_GEMM: role = ROLE_WO; break;
+        case ADN_STAGE_LMHEAD_GEMM: role = ROLE_LMHEAD; N = cfg->vocab; S = 1; break;
+        case ADN_STAGE_READOUT_GEMM: role = ROLE_READOUT; break;
+        default: return fail(ADN_E_INVALID, "stage is not a product");
+    }
+    const GemmBlocks g = gemm_blocks(role, gemm_prec(*cfg), rows, N, d, S, exits != 0);
+    blocks[0] = g.rows;
+    blocks[1] = g.cols;
+    blocks[2] = g.k_waves;
+    blocks[3] = g.pre && stage != ADN_STAGE_HIST_GEMM;
+    return ADN_OK;
+}
+
 int adn_create(const adn_config *cfg, adn_ctx **out) {
     if (!cfg || !out) return fail(ADN_E_INVALID, "null argument");
     *out = nullptr;
@@ -894,10 +925,7 @@ int adn_create(const adn_config *cfg, adn_ctx **out) {
     try {
         c->cfg = *cfg;
         c->D = Dims{cfg->d_r, cfg->h_slots, cfg->vocab, cfg->d_state, cfg->rank, cfg->flags};
-        c->prec = (cfg->flags & ADN_F_GEMM_FP32)     ? PREC_FP32
-                  : (cfg->flags & ADN_F_GEMM_BF16X3) ? PREC_BF16X3
-                  : (cfg->flags & ADN_F_GEMM_BF16)   ? PREC_BF16X1
-                                                     : PREC_F16X3;
+        c->prec = gemm_prec(*cfg);
         ADN_HIP(hipGetDevice(&c->device));
         if (c->device < 0 || c->device >= 256) throw HipError{hipErrorInvalidDevice, "adn_create: device ordinal"};
         c->fuse_mix = cfg->anderson_m >= 3 && update_mix_ok(c->D);

@@ -27,6 +27,13 @@
  *       pooled             [B][T][d]              (deq_forward_pool.wgsl:32-65)
  *       logits             [B][T][V]              (lm_exact_forward.wgsl:21-47)
  *       carrier state      [B][H][d][N]
+ *   - Rounding and the batch: a token's arithmetic does not depend on its row, but the order in
+ *     which a product sums its inner dimension depends on how many rows it has.  Solves that a
+ *     tolerance or the plateau exit may end use one order for 1-4 rows, one for 5-32 and one
+ *     above (rows = tokens of the call; the B of a position in memory mode), so that above 32
+ *     tokens h* and the iteration counts of a sequence are the same bits whatever else is solved
+ *     with it.  Solves of a fixed step count, and the carrier's projections and readout, choose
+ *     among three orders by their sizes; results then agree to fp32 rounding (about 5e-7).
  */
 #ifndef AIDEEN_HIP_H
 #define AIDEEN_HIP_H
@@ -417,6 +424,14 @@ typedef struct adn_profile {
 /* Runs adn_forward_async with a HIP event pair around every kernel launch on the context
  * stream, synchronises, and fills *prof.  Device-memory arguments as adn_forward_async. */
 int adn_profile_forward(adn_ctx *ctx, const adn_run *run, const adn_outputs *out, adn_profile *prof);
+
+/* No counterpart in the reference.  Diagnostics: the blocks on which one of the forward's products
+ * (stage: ADN_STAGE_SIGNAL_GEMM, _QKV_GEMM, _WO_GEMM, _LMHEAD_GEMM, _READOUT_GEMM or _HIST_GEMM)
+ * of `rows` rows runs for this configuration, in a solve that an exit test may end (exits != 0) or
+ * not: blocks[0], blocks[1] = rows and columns of a block, blocks[2] = the waves its inner dimension
+ * is divided over (1: one sum), blocks[3] = 1 where its input arrives split into halves.  So that
+ * tests can state which kernel their sizes reach.  Host-only. */
+int adn_gemm_blocks(const adn_config *cfg, int32_t stage, int32_t rows, int32_t exits, int32_t *blocks);
 
 #ifdef __cplusplus
 }
