@@ -66,9 +66,9 @@ def capture_and_replay(mc, w, B, T, toks):
 
 @pytest.mark.parametrize("anderson_m", [0, 3])
 def test_forward_graph_replays_match_eager(anderson_m):
-    """1200 tokens at d = 512, H = 2, V = 700: the Q|K|V, W_o and LM-head GEMMs on the persistent
-    256x256 tiles (W_o and the LM head reading operands their producers wrote pre-split), the
-    device-side active list, the carrier scan and the readout; with and without Anderson mixing."""
+    """1200 tokens at d = 512, H = 2, V = 700: the Q|K|V, W_o and LM-head GEMMs on the ring kernel's
+    tiles (W_o and the LM head reading operands their producers wrote pre-split), the device-side
+    active list, the carrier scan and the readout; with and without Anderson mixing."""
     log(f"graph capture, canonical forward, anderson m={anderson_m}")
     mc = synth.ModelConfig(d=512, H=2, V=700, N=4, r=32, anderson_m=anderson_m, max_iters=20)
     w = synth.make_weights(mc, seed=5)

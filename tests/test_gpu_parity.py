@@ -142,8 +142,9 @@ def test_variants_match_oracle(oracle_lib, var):
     assert_forward_parity(got, ref, str(var))
 
 
-# More than 512 tokens in flight: the many-token update kernel, whose slot walk is compiled per
-# slot count (1, 2, 4, 8, 16 at d <= 1024; read at run time at d = 2048).
+# 655 tokens: with one and two slots the many-token update kernel (more than 128 tokens per slot), whose
+# slot walk is compiled per slot count; with 16 slots the wave-per-slot form (many tokens of 16 slots:
+# test_gpu_tiles.py).
 MANY = [
     dict(d=64, H=1, V=300, N=1),
     dict(d=64, H=2, V=300, N=4, flags=synth.F_SCAN_SELECTIVE),
@@ -168,8 +169,8 @@ def test_many_token_update_matches_oracle(oracle_lib, var):
 # ArchitectureConfig allows any d_r and h_slots (aideen-core/src/state.rs:7-58); the reference's own
 # benchmark runs d_r = 192 with the default 8 slots (aideen-bench/src/main.rs:36).  Widths other
 # than powers of two run the kernels' bucketed instantiations, slot counts other than powers of
-# two the run-time-H attention.  Few tokens (<= 512) and many tokens take different update
-# kernels; every width bucket (d/64 of 3, 5, 24) appears.
+# two the attention padded to the next one.  Few tokens (up to 128 per slot) and many take different
+# update kernels; every width bucket (d/64 of 3, 5, 24) appears.
 REF_SHAPES = [
     dict(d=192, H=8, V=65, N=1, flags=0, B=3, T=37),                                        # arch_bench shape
     dict(d=192, H=6, V=300, N=4, flags=synth.F_SCAN_SELECTIVE, anderson_m=3, B=3, T=37),
@@ -180,15 +181,15 @@ REF_SHAPES = [
 ]
 
 
-# 1024 tokens at widths >= 512: W_o and the LM head on the 256x256 split tiles, their A operands
-# written pre-split by the attention (each store width: 4, 2 and 1 values per lane, the
-# run-time slot-count attention at H = 6) and by the pool kernel.
+# 1024 tokens at widths >= 512: W_o and the LM head on the 64x128 and 128x128 ring blocks, their A
+# operands written pre-split by the attention (each store width: 4, 2 and 1 values per lane, the
+# padded slot counts 6 and 3) and by the pool kernel.
 PRESPLIT_SHAPES = [
     dict(d=512, H=6, V=600, N=4, flags=synth.F_SCAN_SELECTIVE),
     dict(d=640, H=4, V=600, N=2, flags=synth.F_SCAN_SELECTIVE | synth.F_SCORE_CLAMP4, qk_bias=True),
     dict(d=576, H=2, V=700, N=1, flags=0),
     dict(d=512, H=4, V=600, N=4, flags=synth.F_SCAN_SELECTIVE, sigma=0.7, anderson_m=3),
-    # ragged token count (3 x 400, the last tiles of every GEMM partial), a 3-slot run-time attention
+    # ragged token count (3 x 400, the last tiles of every GEMM partial), a 3-slot padded attention
     dict(d=768, H=3, V=900, N=8, flags=synth.F_SCAN_SELECTIVE | synth.F_RESID_RELRMS, B=3, T=400),
     # a vocabulary just above one 512-column block, Anderson m = 5, the L2 exit
     dict(d=1024, H=2, V=520, N=16, flags=synth.F_SCAN_SELECTIVE | synth.F_RESID_L2, sigma=0.7, anderson_m=5),
@@ -773,9 +774,9 @@ def test_bf16_input_variant_at_size(oracle_lib, name):
             assert top[-1] - top[-2] < 5e-2, f"{ctx}: arg-max differs without a near-tie"
 
 
-# At least 1024 tokens with V >= 512: the 256x256 persistent GEMM tiles (QKV, W_o, W_in, readout
-# and the LM head with its arg-max epilogue where N >= 512) and a carrier scan split into many
-# time chunks, every output of every token against the oracle.
+# At least 1024 tokens with V >= 512: the 64x128 and 128x128 ring blocks of every product and the LM
+# head's arg-max epilogue (the 256x256 ones: test_gpu_persistent_tiles.py) and a carrier scan split
+# into many time chunks, every output of every token against the oracle.
 LARGE = [
     dict(d=128, H=4, V=4096, N=16, flags=synth.F_SCAN_SELECTIVE, B=4, T=512),
     dict(d=512, H=2, V=2048, N=4, flags=synth.F_SCAN_SELECTIVE | synth.F_SCORE_CLAMP4, qk_bias=True, B=2, T=640),
@@ -874,10 +875,10 @@ def test_nonfinite_inputs_report_nonconvergence(oracle_lib, flags):
 
 def test_nonfinite_inputs_on_wide_tiles(oracle_lib):
     """The same non-finite rows among 1024 tokens at d = 512, V = 600: the projections, W_o and
-    the LM head on the 256x256 tiles (W_o's and the head's A written pre-split by the attention
+    the LM head on 64x128 ring blocks (W_o's and the head's A written pre-split by the attention
     and the pool kernel).  The two tokens run to the cap unconverged with non-finite states; the
     other 1022 match the oracle."""
-    log("non-finite inputs on the 256x256 tiles")
+    log("non-finite inputs on the ring tiles")
     mc, w = _small(d=512, H=4, V=600, N=4, flags=synth.F_SCAN_SELECTIVE, max_iters=12)
     B, T = 4, 256
     toks = synth.make_tokens("uniform", B, T, mc.V, seed=14)
@@ -899,7 +900,7 @@ def test_nonfinite_inputs_on_wide_tiles(oracle_lib):
     assert not np.isfinite(got["h_star"][bad]).any()
     assert np.isfinite(got["h_star"][~bad]).all() and got["converged"][~bad].all()
     good = {k: got[k][~bad][None] for k in got}
-    assert_forward_parity(good, {k: ref[k][~bad][None] for k in good}, "finite tokens, 256x256 tiles")
+    assert_forward_parity(good, {k: ref[k][~bad][None] for k in good}, "finite tokens, ring tiles")
 
 
 @pytest.mark.parametrize("B,T", [(2, 300), (3, 53)], ids=["matrix-form", "per-step"])

@@ -124,9 +124,9 @@ def test_random_config_matches_oracle(oracle_lib, seed):
 
 
 def draw_large(seed):
-    """At least 1024 tokens and a vocabulary of at least 512: the persistent 256 x 256 tiles of
-    every product (pre-split W_o and LM-head operands), the many-token update, Anderson's one- or
-    two-pass mixing, and the per-step or matrix-form carrier scan."""
+    """At least 1024 tokens and a vocabulary of at least 512: the ring tiles of every product
+    (pre-split W_o and LM-head operands), the many-token update, Anderson's one- or two-pass
+    mixing, and the per-step or matrix-form carrier scan."""
     rng = np.random.default_rng(2000 + seed)
     d = int(rng.choice([128, 256, 512]))
     H = int(rng.choice([2, 4, 8]))
@@ -163,7 +163,7 @@ def test_random_large_config_matches_oracle(oracle_lib, seed):
 def draw_wide(seed):
     """Rows of 1024 or 1536 floats at >= 1024 tokens with Anderson mixing of depth 3 or 4 at
     tolerance 0: the fused update and mix for wide rows (a lane's elements walked in groups, the
-    rows in LDS) on the 256 x 256 tile paths.  (Depth 5 at these widths leaves up to 15% of the
+    rows in LDS) on the ring tiles.  (Depth 5 at these widths leaves up to 15% of the
     tokens ill-conditioned in the sense below.)"""
     rng = np.random.default_rng(5000 + seed)
     d = int(rng.choice([1024, 1536]))

@@ -69,11 +69,11 @@ def test_operands_beyond_fp16_range(oracle_lib, flags, anderson_m):
 
 
 def test_operands_beyond_fp16_range_wide_tiles(oracle_lib):
-    """The same scaled model with 1024 tokens at d = 512, V = 600: W_o and the LM head run on the
-    256x256 tiles, whose A operands (the slot mix, the normalised pooled row) their producers write
+    """The same scaled model with 1024 tokens at d = 512, V = 600: W_o and the LM head run on 64x128
+    ring tiles, whose A operands (the slot mix, the normalised pooled row) their producers write
     already split into fp16 halves, at the scale the GEMM derives from the h bound (mix) or the
     head's static bound (pooled row)."""
-    log("range guard on the 256x256 tiles: d=512 H=2 V=600, 1024 tokens")
+    log("range guard on the ring tiles: d=512 H=2 V=600, 1024 tokens")
     mc, w = scaled_model(synth.F_SCAN_SELECTIVE, 0, d=512, H=2, V=600)
     B, T = 4, 256
     toks = synth.make_tokens("uniform", B, T, mc.V, seed=6)

@@ -1,6 +1,6 @@
-"""GEMM tile choices below 1024 rows (needs an MI355X): row and column counts on both sides of every
-block edge (32, 64, 128, 256) and slot counts that move the choice between the K-sliced and the ring
-kernels, every output against the oracle."""
+"""GEMM tile choices (needs an MI355X): row and column counts on both sides of every block edge (32, 64,
+128, 256) and slot counts that move the choice between the K-sliced and the ring kernels, every output
+against the oracle.  tests/test_gemm_blocks.py asserts which blocks the sizes reach."""
 import dataclasses
 
 import numpy as np
@@ -8,7 +8,7 @@ import pytest
 
 from aideen_amd import synth
 from aideen_amd.backend import GpuDeqBackend
-from test_gpu_parity import ATOL, RTOL
+from test_gpu_parity import ATOL, RTOL, assert_forward_parity
 
 pytestmark = pytest.mark.gpu
 
@@ -17,12 +17,17 @@ SHAPES = [
     (64, 1, 65, 1, 5),      # fewer steps of K than waves
     (64, 4, 31, 1, 31),     # one partial row block, one partial column block
     (64, 16, 129, 1, 33),   # one row past a 32-row block
+    (256, 8, 300, 1, 24),   # the few-row head's 128-column blocks
     (192, 8, 65, 1, 128),   # whole blocks, narrow head
     (128, 2, 257, 1, 129),  # one row and one column past a block
     (320, 3, 300, 1, 65),   # K not a power of two, H not a power of two
-    (256, 8, 16500, 1, 97),  # a head wide enough for the 256-column blocks, its last partly filled
-    (192, 16, 513, 3, 171),  # 128-row ring blocks
-    (512, 8, 130, 1, 250),  # 64x64 K-sliced W_o, ring Q|K|V
+    (64, 2, 8300, 1, 33),   # the 64x256 head, one row past the few-row kernel and a partial last block
+    (64, 2, 8300, 1, 64),   # the same, whole row blocks
+    (256, 8, 16500, 1, 97),  # a wide head on 128x128 blocks
+    (192, 16, 513, 3, 171),  # 64x128 ring Q|K|V and head, 32x64 K-sliced W_o
+    (512, 8, 130, 1, 250),  # 128x128 ring Q|K|V, 32x64 K-sliced W_o
+    (192, 8, 130, 1, 810),  # 64x64 K-sliced Q|K|V, 64x128 ring W_o
+    (256, 16, 130, 1, 777),  # 128x128 ring W_o
 ]
 
 
@@ -68,10 +73,14 @@ def test_token_limits_match_oracle(d, H, n):
     assert (got["iters"] == 2).all()
 
 
-@pytest.mark.parametrize("shape", [(128, 8, 257, 1, 1500), (256, 16, 1025, 3, 331)], ids=lambda s: "x".join(map(str, s)))
+# 64x128 blocks throughout; Q|K|V alone on 128x256; every product on 128x256
+BF16_SHAPES = [(128, 8, 257, 1, 1500), (256, 16, 1025, 3, 331), (256, 16, 2100, 1, 3001)]
+
+
+@pytest.mark.parametrize("shape", BF16_SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_bf16_blocks_match_fp32_gemms(shape):
-    """bf16-input products on the 128x256 blocks (a partial last row and column block) against the
-    fp32 products of the same model: one bf16 rounding of each operand, 2^-8 relative a product, well
+    """bf16-input products on the ring blocks up to 128x256 (partial last row and column blocks) against
+    the fp32 products of the same model: one bf16 rounding of each operand, 2^-8 relative a product, well
     inside 2e-2 of outputs of order one after two contracting steps."""
     d, H, V, B, T = shape
     toks = synth.make_tokens("uniform", B, T, V, seed=1)
@@ -87,6 +96,25 @@ def test_bf16_blocks_match_fp32_gemms(shape):
         assert np.abs(a[k] - b[k]).max() <= 2e-2 * max(1.0, np.abs(b[k]).max()), k
     lg = a["logits"].reshape(-1, V)
     assert np.array_equal(a["argmax"].ravel(), V - 1 - np.argmax(lg[:, ::-1], axis=1))
+
+
+# more than 128 tokens per slot at 16 slots: the update with a wave per token, unrolled over 16 slots up
+# to 512 floats and walking them at run time beyond, its L2 exit and active list among them
+@pytest.mark.parametrize("d,n,flags,eps", [(64, 2049, 0, 0.0), (128, 2200, synth.F_RESID_L2, 1e-4),
+                                           (512, 2100, 0, 1e-4), (1024, 2050, synth.F_RESID_L2, 1e-4),
+                                           (1024, 2077, 0, 0.0)])
+def test_many_tokens_of_16_slots_match_oracle(d, n, flags, eps):
+    from oracle import pyoracle
+    mc = synth.ModelConfig(d=d, H=16, V=33, N=1, max_iters=20 if eps else 2, eps=eps, flags=flags)
+    w = synth.make_token_sensitive_weights(mc)
+    toks = synth.make_tokens("uniform", 1, n, mc.V, seed=1)
+    be = GpuDeqBackend(mc, 1, n)
+    be.upload_weights(w)
+    got = be.forward(toks, want=("h_star", "iters", "converged"))
+    be.close()
+    ids, inv = np.unique(toks[0], return_inverse=True)
+    ref = pyoracle.Oracle(mc, w).forward(ids[None].astype(np.int32), nthreads=8, want_scan=False)
+    assert_forward_parity({k: v[0] for k, v in got.items()}, {k: ref[k][0][inv] for k in ("h_star", "iters", "converged")})
 
 
 # (d, H, T, few, many): sequences of T tokens solved in batches of `few` and of `many`, both up to 32

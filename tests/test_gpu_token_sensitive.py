@@ -116,7 +116,7 @@ def test_ns_position_permutation_is_bit_exact(kind):
         assert np.array_equal(rb, ra[perm]), f"{kind}: {k} rows do not permute bit for bit"
 
 
-# at least 1024 tokens with V >= 512: the persistent 256x256 tiles of every GEMM role and the LM
+# at least 1024 tokens with V >= 512: the 64x128 and 128x128 ring tiles of every GEMM role and the LM
 # head's arg-max epilogue, a time-chunked carrier; every output of every token
 LARGE_TS = [
     dict(d=128, H=4, V=4096, N=16, flags=synth.F_SCAN_SELECTIVE, B=4, T=512),
