@@ -32,8 +32,10 @@
  *     tolerance or the plateau exit may end use one order for 1-4 rows, one for 5-32 and one
  *     above (rows = tokens of the call; the B of a position in memory mode), so that above 32
  *     tokens h* and the iteration counts of a sequence are the same bits whatever else is solved
- *     with it.  Solves of a fixed step count, and the carrier's projections and readout, choose
- *     among three orders by their sizes; results then agree to fp32 rounding (about 5e-7).
+ *     with it (inputs no larger than the embedding's entries, states within the fp16 range:
+ *     beyond, the batch's largest value scales the operands of all).  Solves of a fixed step
+ *     count, and the carrier's projections and readout, choose their order by their sizes;
+ *     results then agree to fp32 rounding (about 5e-7).
  */
 #ifndef AIDEEN_HIP_H
 #define AIDEEN_HIP_H

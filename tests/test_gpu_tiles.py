@@ -129,8 +129,22 @@ def test_exit_steps_do_not_depend_on_the_batch(shape, flags):
     """Tokens exit on a tolerance: a sequence's fixed points and iteration counts are the same bits
     whatever else is solved beside it, since a residual within rounding of the tolerance would
     otherwise move a token by one update."""
+    check_exit_steps(shape, flags=synth.F_SCAN_SELECTIVE | flags, eps=1e-4)
+
+
+@pytest.mark.parametrize("shape,kw", [
+    ((512, 8, 256, 1, 9), dict(anderson_m=3, sigma=0.7, eps=1e-3)), ((128, 4, 64, 1, 40), dict(anderson_m=4, eps=1e-3)),
+    ((1024, 4, 50, 1, 12), dict(anderson_m=3, eps=1e-3)), ((512, 8, 256, 1, 9), dict(flags=synth.F_RESID_L2, eps=1e-4)),
+    ((512, 8, 256, 1, 9), dict(flags=synth.F_RESID_RELRMS | synth.F_HOMEOSTATIC_EXIT, eps=1e-4)),
+    ((512, 8, 256, 1, 9), dict(flags=synth.F_RESID_RELRMS | synth.F_HOMEOSTATIC_EXIT, eps=0.0)),
+    ((1536, 5, 60, 1, 8), dict(eps=1e-4))], ids=["anderson", "narrow", "wide-anderson", "l2", "plateau", "plateau-alone", "wide"])
+def test_exit_forms_do_not_depend_on_the_batch(shape, kw):
+    check_exit_steps(shape, **kw)
+
+
+def check_exit_steps(shape, **kw):
     d, H, T, few, many = shape
-    mc = synth.ModelConfig(d=d, H=H, V=97, N=1, max_iters=16, eps=1e-4, flags=synth.F_SCAN_SELECTIVE | flags)
+    mc = synth.ModelConfig(d=d, H=H, V=97, N=1, max_iters=16, **kw)
     w = synth.make_token_sensitive_weights(mc)
     toks = synth.make_tokens("uniform", many, T, mc.V, seed=1)
     be = GpuDeqBackend(mc, many, T)
